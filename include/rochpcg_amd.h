@@ -93,7 +93,8 @@ int hpcgx_vectors(const hpcgx_problem* p, void** ptrs);
  * the permutation (not a bijection), the colouring (not proper, colour table
  * or natural order inside a colour wrong), the ELL rows (not exactly the
  * row's in-range 27-point neighbours through perm, in strictly ascending
- * order, split-padded, with the closed-form count), the values (26 / -1 / 0
+ * order, split-padded, with the closed-form count; nor what its row pattern
+ * says), the values (26 / -1 / 0
  * padding in every store, the diagonal arrays), the row descriptors and
  * diag_idx, and -- when check_vectors is set and level is 0 -- b = 26 -
  * (nnz_row - 1), x = 0, xexact = 1; then the stored nonzeros and the rows
@@ -202,6 +203,10 @@ double hpcgx_flops_per_iteration(const hpcgx_problem* p);
  * vectors once (no reference counterpart; the reference's traffic model is
  * ReportResults.cpp:107-138) */
 int hpcgx_iteration_bytes(const hpcgx_problem* p, int mode, double* vcycle_bytes, double* iteration_bytes);
+/* the same with each kernel's own loads: where a level has row patterns
+ * (hpcgx_set_row_patterns) a slot counts its value alone and a row one byte
+ * for its columns and descriptor */
+int hpcgx_stream_bytes(const hpcgx_problem* p, int mode, double* vcycle_bytes, double* iteration_bytes);
 
 /* ---- the reference's natural-order path on the device -------------------- */
 /* Natural row order (GenerateProblem's numbering), the unoptimized operators
@@ -293,6 +298,14 @@ int hpcgx_get_shape(const hpcgx_problem* p, int prec, int level, int op, int* bl
  * column), 1 = row order, k > 1 = k columns per plane where the colour's tiles
  * divide so.  Results do not depend on it.  level -1 applies to all. */
 int hpcgx_set_sweep_columns(hpcgx_problem* p, int level, int columns);
+/* Where the operators read a level's columns (no reference counterpart; a
+ * tuning knob).  on 1 (the default) = from the level's row patterns -- one byte
+ * a row naming one of its colour's lists of 27 column offsets, built at setup
+ * from the column array -- where the level has them; 0 = from the column
+ * array.  Results do not depend on it.  A level has row patterns when each of
+ * its colours repeats at most 32 lists, as the parity colourings of even grids
+ * do; other levels always read the column array.  level -1 applies to all. */
+int hpcgx_set_row_patterns(hpcgx_problem* p, int level, int on);
 int hpcgx_synchronize(hpcgx_problem* p);
 int hpcgx_malloc(void** ptr, size_t bytes);
 int hpcgx_free(void* ptr);

@@ -85,9 +85,11 @@ def _load():
         "hpcgx_cg_ref": ([vp, vp, vp, i32, f64, i32, P(i32), P(f64), P(f64), vp, i32, vp], i32),
         "hpcgx_flops_per_iteration": ([vp], f64),
         "hpcgx_iteration_bytes": ([vp, i32, P(f64), P(f64)], i32),
+        "hpcgx_stream_bytes": ([vp, i32, P(f64), P(f64)], i32),
         "hpcgx_time_operator": ([vp, i32, i32, i32, i32, P(f64)], i32),
         "hpcgx_set_shape": ([vp, i32, i32, i32, i32, i32], i32),
         "hpcgx_set_sweep_columns": ([vp, i32, i32], i32),
+        "hpcgx_set_row_patterns": ([vp, i32, i32], i32),
         "hpcgx_get_shape": ([vp, i32, i32, i32, P(i32), P(i32)], i32),
         "hpcgx_synchronize": ([vp], i32),
         "hpcgx_batch_create": ([i32, vp, i32, i32, vp, P(vp)], i32),
@@ -414,6 +416,11 @@ class Problem:
         order, k > 1 sweeps k columns per plane (results do not change)."""
         _check(lib.hpcgx_set_sweep_columns(self.h, level, columns))
 
+    def set_row_patterns(self, on, level=-1):
+        """Read columns from the row patterns (True) or from the column array
+        (False) where a level has both (results do not change)."""
+        _check(lib.hpcgx_set_row_patterns(self.h, level, int(bool(on))))
+
     def get_shape(self, level, op, mixed=False):
         b, r = C.c_int(), C.c_int()
         _check(lib.hpcgx_get_shape(self.h, int(mixed), level, op, C.byref(b), C.byref(r)))
@@ -490,6 +497,13 @@ class Problem:
         """Algorithmic HBM bytes (V-cycle, whole CG iteration) of this library's kernels."""
         mg, it = C.c_double(), C.c_double()
         _check(lib.hpcgx_iteration_bytes(self.h, mode, C.byref(mg), C.byref(it)))
+        return mg.value, it.value
+
+    def stream_bytes(self, mode=CG_F64):
+        """The same as the kernels load it: row patterns instead of columns
+        where a level has them."""
+        mg, it = C.c_double(), C.c_double()
+        _check(lib.hpcgx_stream_bytes(self.h, mode, C.byref(mg), C.byref(it)))
         return mg.value, it.value
 
     def time_operator(self, op, level=0, mixed=False, reps=10):

@@ -12,6 +12,7 @@
 // (kernels.hpp), so each problem computes exactly what it would alone, up to
 // the grouping of the dot-product partials.
 #include "batch.hpp"
+#include "batch_rows.hpp"
 #include "kernels.hpp"
 #include "setup.hpp"
 
@@ -22,112 +23,14 @@
 namespace hpcgx
 {
 
-// the fold of a reducing launch: block k folds segment k's partials (one per
-// block of the segment) for that segment's problem
+// the fold of a reducing launch: block k folds the partials of segment k's
+// problem (one per block of the problem's segments) if k is its first segment
 template <int BS>
 __global__ __launch_bounds__(BS) void kb_fold(const BSeg* __restrict__ segs)
 {
     const BSeg& S = segs[blockIdx.x];
-    if(gated(S.gate) || S.ra.partial == nullptr) return;
-    fold_partials<BS>(S.ra.partial, S.nblk, S.ra);
-}
-
-#define BSEG()                                                \
-    const int64_t b_ = xcd_block(blockIdx.x, gridDim.x);      \
-    const BSeg& S = segs[seg_map(segs, nseg)[b_]];            \
-    if(gated(S.gate)) return;                                 \
-    const int64_t lb = b_ - S.blk0;
-
-template <typename VT, typename XT, typename YT, bool DOT, int BS>
-__global__ __launch_bounds__(BS) void kb_spmv(const BSeg* __restrict__ segs, int nseg)
-{
-    BSEG();
-    const int64_t i = lb * BS + threadIdx.x;
-    double acc = 0.0;
-    if(i < S.size)
-    {
-        const int64_t row = S.off + i;
-        XT s[1];
-        row_spmv<VT, XT, 1>(row, S.col, (const VT*)S.val, (const XT*)S.r, s);
-        ((YT*)S.x)[row] = (YT)s[0];
-        if(DOT) acc = fmaT((double)((const XT*)S.r)[row], (double)s[0], acc);
-    }
-    if(DOT) block_partial<BS>(acc, S.ra.partial, lb);
-}
-
-// The sweeps are compiled for the widest window of the launch's segments
-// (BLaunch::win), like the single-problem kernels, and for R rows per thread
-// (BLaunch::rows; 2 only when every segment's offset and size are even).
-template <int NS, typename VT, typename XT, typename RT, int R, int BS>
-__global__ __launch_bounds__(BS) void kb_fwd_zero(const BSeg* __restrict__ segs, int nseg)
-{
-    BSEG();
-    const int64_t i = (lb * BS + threadIdx.x) * R;
-    if(i >= S.size) return;
-    row_fwd_zero<NS, VT, XT, RT, R>(S.off + i, S.col, (const VT*)S.val, (const VT*)S.dg, S.desc,
-                                    (const RT*)S.r, (XT*)S.x);
-}
-
-template <int NS, typename VT, typename XT, int R, int BS>
-__global__ __launch_bounds__(BS) void kb_bwd_zero(const BSeg* __restrict__ segs, int nseg)
-{
-    BSEG();
-    const int64_t i = (lb * BS + threadIdx.x) * R;
-    if(i >= S.size) return;
-    if(S.t)
-        row_bwd_zero<NS, VT, XT, true, R>(S.off + i, S.col, (const VT*)S.val, (const VT*)S.dg, S.desc,
-                                          (XT*)S.x, (XT*)S.t);
-    else
-        row_bwd_zero<NS, VT, XT, false, R>(S.off + i, S.col, (const VT*)S.val, (const VT*)S.dg, S.desc,
-                                           (XT*)S.x, nullptr);
-}
-
-// every segment reuses its pre-smoother's upper sums (BLaunch::all_u)
-template <int NA, int NB, typename VT, typename XT, typename RT, int R, int BS>
-__global__ __launch_bounds__(BS) void kb_fwd_full_u(const BSeg* __restrict__ segs, int nseg)
-{
-    BSEG();
-    const int64_t i = (lb * BS + threadIdx.x) * R;
-    if(i >= S.size) return;
-    row_fwd_full_u<NA, NB, VT, XT, RT, R>(S.off + i, S.col, (const VT*)S.val, (const VT*)S.dg, S.desc,
-                                          (const RT*)S.r, (XT*)S.x, (XT*)S.t);
-}
-
-template <typename VT, typename XT, typename RT, int R, int BS>
-__global__ __launch_bounds__(BS) void kb_fwd_full(const BSeg* __restrict__ segs, int nseg)
-{
-    BSEG();
-    const int64_t i = (lb * BS + threadIdx.x) * R;
-    if(i >= S.size) return;
-    if(S.use_u)
-        row_fwd_full_u<W - 1, W - 1, VT, XT, RT, R>(S.off + i, S.col, (const VT*)S.val, (const VT*)S.dg,
-                                                    S.desc, (const RT*)S.r, (XT*)S.x, (XT*)S.t);
-    else if(S.t)
-        row_fwd_full<VT, XT, RT, true, R>(S.off + i, S.col, (const VT*)S.val, (const RT*)S.r, (XT*)S.x,
-                                          (XT*)S.t);
-    else
-        row_fwd_full<VT, XT, RT, false, R>(S.off + i, S.col, (const VT*)S.val, (const RT*)S.r, (XT*)S.x,
-                                           nullptr);
-}
-
-template <int NS, typename VT, typename XT, int R, int BS>
-__global__ __launch_bounds__(BS) void kb_bwd_full(const BSeg* __restrict__ segs, int nseg)
-{
-    BSEG();
-    const int64_t i = (lb * BS + threadIdx.x) * R;
-    if(i >= S.size) return;
-    row_bwd_full<NS, VT, XT, R>(S.off + i, S.col, (const VT*)S.val, (const VT*)S.dg, S.desc,
-                                (const XT*)S.t, (XT*)S.x);
-}
-
-template <typename VT, typename XT, typename RT, int BS>
-__global__ __launch_bounds__(BS) void kb_restrict(const BSeg* __restrict__ segs, int nseg)
-{
-    BSEG();
-    const int64_t k = lb * BS + threadIdx.x;
-    if(k >= S.size) return;
-    row_restrict<VT, XT, RT, XT>(k, S.col, (const VT*)S.val, S.f2c_fine, S.f2c_coarse, (const RT*)S.r,
-                                 (const XT*)S.x, (XT*)S.rc);
+    if(gated(S.gate) || S.ra.partial == nullptr || S.nfold == 0) return;
+    fold_partials<BS>(S.ra.partial, S.nfold, S.ra);
 }
 
 template <typename XT, int BS>
@@ -156,7 +59,7 @@ __global__ __launch_bounds__(BS) void kb_dot(const BSeg* __restrict__ segs, int 
     const YT* bb = (const YT*)S.b;
     double acc = 0.0;
     for(int64_t i = e0 + threadIdx.x; i < e1; i += BS) acc = fmaT((double)bb[i], (double)a[i], acc);
-    block_partial<BS>(acc, S.ra.partial, lb);
+    block_partial<BS>(acc, S.ra.partial, S.part0 + lb);
 }
 
 template <typename ZT, int BS>
@@ -189,7 +92,7 @@ __global__ __launch_bounds__(BS) void kb_cg_xr(const BSeg* __restrict__ segs, in
         x[i] = fmaT(alpha, p[i], x[i]);
         acc = fmaT(rv, rv, acc);
     }
-    block_partial<BS>(acc, S.ra.partial, lb);
+    block_partial<BS>(acc, S.ra.partial, S.part0 + lb);
 }
 
 template <int BS>
@@ -213,20 +116,10 @@ __global__ __launch_bounds__(BS) void kb_waxpby(const BSeg* __restrict__ segs, i
     double* w = (double*)S.w;
     for(int64_t i = e0 + threadIdx.x; i < e1; i += BS) w[i] = fmaT(beta, bb[i], a[i]);
 }
-#undef BSEG
 #undef BCHUNK
 
 // ---------------------------------------------------------------------------
 // launching a planned record
-
-template <typename F>
-static void with_rows(int rows, F&& f)
-{
-    if(rows == 2)
-        f(std::integral_constant<int, 2>{});
-    else
-        f(std::integral_constant<int, 1>{});
-}
 
 template <int BS>
 static void launch_bs(const BLaunch& L, hipStream_t s)
@@ -237,92 +130,6 @@ static void launch_bs(const BLaunch& L, hipStream_t s)
     const bool f64 = L.prec == PREC_F64;
     switch(L.kind)
     {
-    case BK_SPMV:
-        // outer SpMV: f64 vectors over either store; MG-internal SpMV is not batched
-        if(f64)
-        {
-            if(L.dot)
-                hipLaunchKernelGGL((kb_spmv<double, double, double, true, BS>), g, b, 0, s, T, n);
-            else
-                hipLaunchKernelGGL((kb_spmv<double, double, double, false, BS>), g, b, 0, s, T, n);
-        }
-        else
-        {
-            if(L.dot)
-                hipLaunchKernelGGL((kb_spmv<__half, double, double, true, BS>), g, b, 0, s, T, n);
-            else
-                hipLaunchKernelGGL((kb_spmv<__half, double, double, false, BS>), g, b, 0, s, T, n);
-        }
-        break;
-    case BK_FWD_ZERO:
-        with_rows(L.rows, [&](auto RR) {
-            constexpr int R = decltype(RR)::value;
-            with_window(L.win, [&](auto NN) {
-                constexpr int NS = decltype(NN)::value;
-                if(f64)
-                    hipLaunchKernelGGL((kb_fwd_zero<NS, double, double, double, R, BS>), g, b, 0, s, T, n);
-                else if(L.r_f64)
-                    hipLaunchKernelGGL((kb_fwd_zero<NS, __half, float, double, R, BS>), g, b, 0, s, T, n);
-                else
-                    hipLaunchKernelGGL((kb_fwd_zero<NS, __half, float, float, R, BS>), g, b, 0, s, T, n);
-            });
-        });
-        break;
-    case BK_BWD_ZERO:
-        with_rows(L.rows, [&](auto RR) {
-            constexpr int R = decltype(RR)::value;
-            with_window(L.win, [&](auto NN) {
-                constexpr int NS = decltype(NN)::value;
-                if(f64)
-                    hipLaunchKernelGGL((kb_bwd_zero<NS, double, double, R, BS>), g, b, 0, s, T, n);
-                else
-                    hipLaunchKernelGGL((kb_bwd_zero<NS, __half, float, R, BS>), g, b, 0, s, T, n);
-            });
-        });
-        break;
-    case BK_FWD_FULL:
-        with_rows(L.rows, [&](auto RR) {
-            constexpr int R = decltype(RR)::value;
-            if(L.all_u)
-                with_window_pair(L.win, L.win_tail, [&](auto NA_, auto NB_) {
-                    constexpr int NA = decltype(NA_)::value, NB = decltype(NB_)::value;
-                    if(f64)
-                        hipLaunchKernelGGL((kb_fwd_full_u<NA, NB, double, double, double, R, BS>), g, b, 0, s, T,
-                                           n);
-                    else if(L.r_f64)
-                        hipLaunchKernelGGL((kb_fwd_full_u<NA, NB, __half, float, double, R, BS>), g, b, 0, s, T,
-                                           n);
-                    else
-                        hipLaunchKernelGGL((kb_fwd_full_u<NA, NB, __half, float, float, R, BS>), g, b, 0, s, T, n);
-                });
-            else if(f64)
-                hipLaunchKernelGGL((kb_fwd_full<double, double, double, R, BS>), g, b, 0, s, T, n);
-            else if(L.r_f64)
-                hipLaunchKernelGGL((kb_fwd_full<__half, float, double, R, BS>), g, b, 0, s, T, n);
-            else
-                hipLaunchKernelGGL((kb_fwd_full<__half, float, float, R, BS>), g, b, 0, s, T, n);
-        });
-        break;
-    case BK_BWD_FULL:
-        with_rows(L.rows, [&](auto RR) {
-            constexpr int R = decltype(RR)::value;
-            with_window(L.win, [&](auto NN) {
-                constexpr int NS = decltype(NN)::value;
-                if(f64)
-                    hipLaunchKernelGGL((kb_bwd_full<NS, double, double, R, BS>), g, b, 0, s, T, n);
-                else
-                    hipLaunchKernelGGL((kb_bwd_full<NS, __half, float, R, BS>), g, b, 0, s, T, n);
-            });
-        });
-        break;
-    case BK_RESTRICT:
-        if(f64)
-            hipLaunchKernelGGL((kb_restrict<double, double, double, BS>), g, b, 0, s, T, n);
-        else if(L.r_f64)
-            hipLaunchKernelGGL((kb_restrict<__half, float, double, BS>), g, b, 0, s, T, n);
-        else
-            hipLaunchKernelGGL((kb_restrict<__half, float, float, BS>), g, b, 0, s, T, n);
-        break;
     case BK_PROLONG:
         if(f64)
             hipLaunchKernelGGL((kb_prolong<double, BS>), g, b, 0, s, T, n);
@@ -350,12 +157,14 @@ static void launch_bs(const BLaunch& L, hipStream_t s)
 static int launch(const BLaunch& L, hipStream_t s)
 {
     if(L.nblocks == 0) return 0;
-    switch(L.block)
-    {
-    case 64: launch_bs<64>(L, s); break;
-    case 128: launch_bs<128>(L, s); break;
-    default: launch_bs<256>(L, s); break;
-    }
+    if(L.kind <= BK_RESTRICT)
+        HPCGX_TRY(L.pat ? launch_batch_rows<true>(L, s) : launch_batch_rows<false>(L, s));
+    else if(L.block == 64)
+        launch_bs<64>(L, s);
+    else if(L.block == 128)
+        launch_bs<128>(L, s);
+    else
+        launch_bs<256>(L, s);
     HPCGX_HIP(hipGetLastError());
     if(L.kind == BK_DOT || L.kind == BK_CG_XR || (L.kind == BK_SPMV && L.dot))
     {
@@ -378,6 +187,8 @@ struct Planner
     int next_win = W, next_tail = W, next_all_u = 0;
     // rows per thread of the next sweep launch (2 needs even segment offsets and sizes)
     int next_rows = 1;
+    // segments per problem of the next launch, and the one being filled
+    int next_subs = 1, sub = 0;
 
     // widest window of kind `wk` of colour c on level l over the problems
     // that have the colour
@@ -396,22 +207,32 @@ struct Planner
         std::vector<BSeg> segs;
         std::vector<size_t> prob;
         for(size_t k = 0; k < B.probs.size(); ++k)
-        {
-            BSeg sg;
-            std::memset(&sg, 0, sizeof(sg));
-            sg.gate = &B.probs[k]->sc->done;
-            if(!fill((int)k, sg) || sg.size <= 0) continue;
-            segs.push_back(sg);
-            prob.push_back(k);
-        }
+            for(sub = 0; sub < next_subs; ++sub)
+            {
+                BSeg sg;
+                std::memset(&sg, 0, sizeof(sg));
+                sg.gate = &B.probs[k]->sc->done;
+                if(!fill((int)k, sg) || sg.size <= 0) continue;
+                segs.push_back(sg);
+                prob.push_back(k);
+            }
         const int rows = launch_rows(segs.data(), segs.size(), next_rows);
         const int64_t nb = assign_blocks(segs.data(), segs.size(), block, vector_kind, rows);
-        for(size_t j = 0; j < segs.size(); ++j)
-            if(segs[j].ra.partial && segs[j].nblk > B.probs[prob[j]]->partial_cap)
+        // the segments of a problem follow each other: their partials too, and
+        // the first folds them all
+        int pat = kind <= BK_RESTRICT;
+        for(size_t j = 0, first = 0; j < segs.size(); ++j)
+        {
+            if(prob[j] != prob[first]) first = j;
+            segs[j].part0 = segs[first].nfold;
+            segs[first].nfold += segs[j].nblk;
+            if(segs[j].ra.partial && segs[first].nfold > B.probs[prob[j]]->partial_cap)
             {
                 set_error("batched reduction exceeds the partial capacity");
                 return -2;
             }
+            if(!segs[j].cols.pat) pat = 0;
+        }
         BLaunch L;
         std::memset(&L, 0, sizeof(L));
         for(const BSeg& sg : segs)
@@ -432,6 +253,8 @@ struct Planner
         L.win_tail = next_tail;
         L.all_u = next_all_u;
         L.rows = rows;
+        L.pat = pat;
+        next_subs = 1;
         next_bf32 = 0;
         next_win = next_tail = W;
         next_all_u = 0;
@@ -471,6 +294,12 @@ struct Planner
 
     const void* vals(const Level& L) { return prec == PREC_F64 ? (const void*)L.ell_val : (const void*)L.ell_h; }
     const void* diags(const Level& L) { return prec == PREC_F64 ? (const void*)L.diag64 : (const void*)L.diag_h; }
+    ColArgs columns(const Level& L, int c)
+    {
+        ColArgs a = L.cols(c);
+        if(!L.use_pat()) a.pat = nullptr;
+        return a;
+    }
     LevelVecs* vecs(Problem* P) { return prec == PREC_F64 ? P->v64 : P->v32; }
     void* z(Problem* P) { return prec == PREC_F64 ? (void*)P->z64 : (void*)P->z32; }
 
@@ -493,9 +322,8 @@ struct Planner
             if(c >= L.ncolors) return false;
             s.off = L.offsets[c];
             s.size = L.sizes[c];
-            s.col = L.ell_col;
+            s.cols = columns(L, c);
             s.val = vals(L);
-            s.desc = L.desc;
             s.dg = diags(L);
             s.r = (l == 0) ? (const void*)P->r : vecs(P)[l].r;
             s.x = (l == 0) ? z(P) : vecs(P)[l].x;
@@ -525,7 +353,8 @@ struct Planner
             Problem* P = B.probs[k];
             const Level& L = P->L[l];
             s.size = L.mc;
-            s.col = L.ell_col;
+            s.cols = columns(L, L.ncolors - 1);
+            if(!L.u_ok) s.cols.pat = nullptr;   // injected rows of several colours
             s.val = vals(L);
             s.f2c_fine = L.f2c_fine;
             s.f2c_coarse = L.f2c_coarse;
@@ -580,12 +409,14 @@ struct Planner
 
     int outer_spmv(bool dot, bool from_x, bool into_tmp)
     {
+        next_subs = max_colors(0);   // one segment per colour: a block stages one colour's patterns
         return add(BK_SPMV, B.block[0], false, 1, dot ? 1 : 0, 0.0, [&](int k, BSeg& s) {
             Problem* P = B.probs[k];
             const Level& L = P->L[0];
-            s.off = 0;
-            s.size = L.m;
-            s.col = L.ell_col;
+            if(sub >= L.ncolors) return false;
+            s.off = L.offsets[sub];
+            s.size = L.sizes[sub];
+            s.cols = columns(L, sub);
             s.val = vals(L);
             s.r = from_x ? (const void*)P->x : (const void*)P->p;
             s.x = into_tmp ? (void*)P->tmp : (void*)P->Ap;
@@ -767,7 +598,7 @@ static int run_list(const std::vector<BLaunch>& v, hipStream_t s)
 }
 
 // algorithmic HBM bytes of one planned launch (the per-row model of
-// iteration_bytes in solver.hip, over the launch's rows)
+// iteration_bytes in solver.hip by the ELL's bytes, over the launch's rows)
 static double launch_bytes(const BLaunch& L)
 {
     const bool f64 = L.prec == PREC_F64;

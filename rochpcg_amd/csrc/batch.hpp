@@ -16,9 +16,10 @@ struct BSeg
     int64_t nblk;      // blocks of the segment
     int64_t off;       // first row (or element) of the segment
     int64_t size;      // rows (or elements) in the segment
-    const int32_t* col;
+    int64_t part0;     // reductions: the segment's first partial slot ...
+    int64_t nfold;     // ... and, on its problem's first segment, the partials to fold
+    ColArgs cols;      // columns and descriptors (pat null: the column array)
     const void* val;
-    const int32_t* desc;   // row descriptors (Level::desc)
     const void* dg;    // diagonal values (Level::diag64 / diag_h)
     const void* r;     // rhs / first vector operand
     void* x;           // solution / in-out operand
@@ -117,6 +118,7 @@ struct BLaunch
     int win_tail;     // post-smoother forward sweep: widest last-colour window
     int all_u;        // post-smoother forward sweep: every segment reuses its upper sums
     int rows;         // sweeps: rows per thread (1 or 2)
+    int pat;          // row kernels: every segment has row patterns
     int nseg;
     int64_t nblocks;
     BSeg* segs;       // device table

@@ -472,7 +472,7 @@ double hpcgx_flops_per_iteration(const hpcgx_problem* p)
     return hpcg_flops_per_iter(*p->P);
 }
 
-int hpcgx_iteration_bytes(const hpcgx_problem* p, int mode, double* vcycle_bytes, double* iteration_bytes)
+static int bytes_of(const hpcgx_problem* p, int mode, bool stream, double* vcycle_bytes, double* iteration_bytes)
 {
     CHECK_P(p);
     if(mode != CG_F64 && mode != CG_MIXED)
@@ -480,7 +480,17 @@ int hpcgx_iteration_bytes(const hpcgx_problem* p, int mode, double* vcycle_bytes
         set_error("invalid CG mode");
         return -2;
     }
-    return hpcgx::iteration_bytes(*p->P, mode, vcycle_bytes, iteration_bytes);
+    return hpcgx::iteration_bytes(*p->P, mode, stream, vcycle_bytes, iteration_bytes);
+}
+
+int hpcgx_iteration_bytes(const hpcgx_problem* p, int mode, double* vcycle_bytes, double* iteration_bytes)
+{
+    return bytes_of(p, mode, false, vcycle_bytes, iteration_bytes);
+}
+
+int hpcgx_stream_bytes(const hpcgx_problem* p, int mode, double* vcycle_bytes, double* iteration_bytes)
+{
+    return bytes_of(p, mode, true, vcycle_bytes, iteration_bytes);
 }
 
 // ---------------------------------------------------------------------------
@@ -586,6 +596,20 @@ int hpcgx_set_sweep_columns(hpcgx_problem* p, int level, int columns)
     for(int l = 0; l < p->P->nlevels; ++l)
         if(level < 0 || l == level) p->P->L[l].zcols = columns;
     // a captured CG iteration keeps the block order it was captured with
+    p->P->invalidate_graphs();
+    return 0;
+}
+
+int hpcgx_set_row_patterns(hpcgx_problem* p, int level, int on)
+{
+    CHECK_P(p);
+    if((on != 0 && on != 1) || level < -1 || level >= p->P->nlevels)
+    {
+        set_error("invalid level or row-pattern choice");
+        return -2;
+    }
+    for(int l = 0; l < p->P->nlevels; ++l)
+        if(level < 0 || l == level) p->P->L[l].pat_off = on == 0;
     p->P->invalidate_graphs();
     return 0;
 }

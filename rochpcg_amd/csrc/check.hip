@@ -40,6 +40,9 @@ struct CheckLevel
     const int32_t* perm;
     const int32_t* colors;
     const int32_t* col;
+    const uint8_t* pat;
+    const int32_t* pat_tab;
+    int npat;
     const double* val;      // may be null
     const __half* val_h;    // may be null
     const int32_t* diag_idx;
@@ -175,6 +178,15 @@ __global__ __launch_bounds__(256) void k_check_rows(CheckLevel L, const int32_t*
                 if(L.diag64 && L.diag64[r] != 26.0) e[CHECK_VALUE]++;
                 if(L.inv_diag && L.inv_diag[r] != 1.0 / 26.0) e[CHECK_VALUE]++;
                 if(L.diag_h && __half2float(L.diag_h[r]) != 26.0f) e[CHECK_VALUE]++;
+                // the row's pattern gives the same columns and descriptor
+                if(L.pat)
+                {
+                    const int id = L.pat[r];
+                    const int32_t* t = L.pat_tab + ((int64_t)c * PAT_MAX + (id < L.npat ? id : 0)) * (PAT_QUADS * 4);
+                    bool same = id < L.npat && t[W] == L.desc[r];
+                    for(int p = 0; p < W; ++p) same = same && t[p] == (cc[p] < 0 ? 0 : cc[p] - (int32_t)r);
+                    if(!same) e[CHECK_ELL]++;
+                }
                 const int32_t ds = L.desc[r];
                 if(L.diag_idx[r] != d || (ds & 255) != d || ((ds >> 8) & 255) != tl || ((ds >> 16) & 255) != us)
                     e[CHECK_DESC]++;
@@ -215,6 +227,9 @@ int check_problem(const Level& L, const double* b, const double* x, const double
     C.perm = L.perm;
     C.colors = L.colors;
     C.col = L.ell_col;
+    C.pat = L.pat;
+    C.pat_tab = L.pat_tab;
+    C.npat = L.npat;
     C.val = L.ell_val;
     C.val_h = L.ell_h;
     C.diag_idx = L.diag_idx;

@@ -82,6 +82,23 @@ enum WinKind : int
     WIN_COUNT = 3
 };
 
+// Row patterns of a level (Cols<true> in kernels.hpp): a pattern is the 27
+// column offsets of a row (column - row, 0 in unused slots) and its
+// descriptor, PAT_QUADS int4 in all; a colour keeps at most PAT_MAX of them.
+constexpr int PAT_MAX = 32;
+constexpr int PAT_QUADS = (W + 1) / 4;
+static_assert(PAT_QUADS * 4 == W + 1, "27 offsets and the descriptor fill whole int4s");
+
+// Where a kernel finds the columns and descriptors of one colour's rows.
+struct ColArgs
+{
+    const int32_t* col;    // column array and row descriptors
+    const int32_t* desc;
+    const uint8_t* pat;    // pattern of each row of the level
+    const int32_t* tab;    // the colour's patterns
+    int npat;              // patterns to stage
+};
+
 // tunable operators of a level.  A sweep has two shapes: one for its wide
 // colours (slot window over 16) and one (SH_NARROW + op) for the others.
 enum ShapeOp : int
@@ -119,6 +136,12 @@ struct Level
     __half* ell_h = nullptr;      // [W*ell_rows(m)] (mixed levels)
     int32_t* diag_idx = nullptr;  // [m] slot of the diagonal
     int32_t* desc = nullptr;      // [m] row descriptor: diagonal slot, first last-colour slot, first upper slot
+    // row patterns (null: the rows repeat too little, or the level is too
+    // large for 32-bit gather offsets); derived from ell_col and desc
+    uint8_t* pat = nullptr;       // [m] pattern of each row, within its colour
+    int32_t* pat_tab = nullptr;   // [ncolors][PAT_MAX][PAT_QUADS*4]
+    int npat = 0;                 // patterns of the colour that has most
+    bool pat_off = false;         // the kernels read the column array all the same
     double* inv_diag = nullptr;   // [m] 1/a_ii (f64)
     double* diag64 = nullptr;     // [m] a_ii (f64 levels)
     __half* diag_h = nullptr;     // [m] a_ii (mixed levels)
@@ -141,6 +164,12 @@ struct Level
     int zcols = 0;
 
     Shape shp[2][SH_COUNT];   // [precision][operator]
+
+    bool use_pat() const { return pat != nullptr && !pat_off; }
+    ColArgs cols(int c) const
+    {
+        return ColArgs{ell_col, desc, pat, pat_tab ? pat_tab + (int64_t)c * PAT_MAX * PAT_QUADS * 4 : nullptr, npat};
+    }
 };
 
 // Device-side CG scalars (one cache line each to avoid false sharing is not

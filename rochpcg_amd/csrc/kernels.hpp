@@ -241,35 +241,7 @@ struct Tiles
 };
 
 // ---------------------------------------------------------------------------
-// Row bodies shared by the single-problem kernels (ops.hip) and the batched
-// kernels (batch.hip).  A thread owns rows [row, row+R) (R-aligned).
-
-// y = A x on R rows; returns the row sums in s[].
-template <typename VT, typename XT, int R>
-__device__ __forceinline__ void row_spmv(int64_t row, const int32_t* __restrict__ col,
-                                         const VT* __restrict__ val, const XT* __restrict__ x, XT (&s)[R])
-{
-    int32_t cc[W][R];
-    VT av[W][R];
-#pragma unroll
-    for(int p = 0; p < W; ++p) ld_nt<R>(col + ell_at(p, row), cc[p]);
-#pragma unroll
-    for(int p = 0; p < W; ++p) ld_nt<R>(val + ell_at(p, row), av[p]);
-    XT xv[W][R];
-#pragma unroll
-    for(int p = 0; p < W; ++p)
-#pragma unroll
-        for(int k = 0; k < R; ++k) xv[p][k] = (cc[p][k] >= 0) ? x[cc[p][k]] : (XT)0;
-#pragma unroll
-    for(int k = 0; k < R; ++k) s[k] = 0;
-#pragma unroll
-    for(int p = 0; p < W; ++p)
-#pragma unroll
-        for(int k = 0; k < R; ++k)
-            if(cc[p][k] >= 0) s[k] = fmaT(cvt<XT>(av[p][k]), xv[p][k], s[k]);
-}
-
-// ELL layout of the sweeps ("split" padding).  The entries of a row keep
+// ELL layout of the rows ("split" padding).  The entries of a row keep
 // the ascending multicolour column order of the reference's ELL, but the
 // padding sits between the diagonal and the upper entries instead of at the
 // tail: slots [0, d) hold the lower entries, slot d the diagonal, slots
@@ -277,7 +249,7 @@ __device__ __forceinline__ void row_spmv(int64_t row, const int32_t* __restrict_
 // largest columns) are their tail [tl, W).  Every window a sweep reads then
 // starts at a slot that does not depend on the row -- 0 for the lower
 // entries, W - NS for the upper or last-colour ones -- so its loads are issued
-// with the row's descriptor load instead of after it.
+// before anything about the row is known.
 //
 // Row descriptor, one int32 per row: bits 0-7 the diagonal slot d, bits 8-15
 // the first slot of an off-diagonal last-colour column tl, bits 16-23 the
@@ -297,36 +269,152 @@ __device__ __forceinline__ int desc_upper(int32_t v) { return (v >> 16) & 255; }
 // then keep one unused element.
 constexpr int slot_dim(int n) { return n > 0 ? n : 1; }
 
-template <int NS, typename VT, int R>
-__device__ __forceinline__ void load_window(int64_t row, const int32_t* __restrict__ col,
-                                            const VT* __restrict__ val, int start,
-                                            int32_t (&cc)[slot_dim(NS)][R], VT (&av)[slot_dim(NS)][R])
-{
-#pragma unroll
-    for(int q = 0; q < NS; ++q)
-    {
-        ld_nt<R>(col + ell_at(start + q, row), cc[q]);
-        ld_nt<R>(val + ell_at(start + q, row), av[q]);
-    }
-}
+// Column sources.  A row body takes the columns and the descriptor of its R
+// rows from one of two places:
+//
+//   PAT = false  the level's ELL column array and descriptors (4 B a slot);
+//   PAT = true   the level's row patterns (Level::pat): one byte a row names a
+//                pattern of its colour, and the pattern holds the 27 column
+//                offsets (column - row) and the descriptor.
+//
+// Why patterns: with f64 values a slot streams 12 B, 4 of them the column;
+// with f16 values 6 B, 4 of them the column -- yet the rows of a colour repeat
+// a handful of offset lists.  The patterns are found from the ELL itself at
+// setup (build_patterns), for whatever matrix it holds; a level whose rows
+// repeat too little keeps its column array.  The offsets are exact, so both
+// sources give the same x values in the same slots and every sum is the same
+// bit for bit.
+//
+// The colour's patterns (112 B each) are staged in LDS by the block while the
+// value loads are in flight, so the x gathers wait for one byte load and an
+// LDS read instead of for the whole column stream.  Gather offsets are 32-bit
+// byte offsets from x (one add-shift a slot); build_patterns keeps levels of
+// 2^29 rows or more on the column array.
+template <bool PAT, int R, int BS>
+struct Cols;
 
-// Neighbour values of every loaded slot with a column (a slot the row does
-// not use reads a value that is then ignored: its own diagonal, or a
-// neighbour outside the window's kind -- never a row this launch writes).
-template <int NS, typename XT, int R>
-__device__ __forceinline__ void gather(const int32_t (&cc)[slot_dim(NS)][R], const XT* __restrict__ x,
-                                       XT (&xv)[slot_dim(NS)][R])
+template <int R, int BS>
+struct Cols<false, R, BS>
+{
+    template <int NS>
+    struct Win
+    {
+        int32_t c[slot_dim(NS)][R];
+    };
+    const ColArgs& a;
+    int64_t row;
+    int32_t ds[R];
+    __device__ __forceinline__ Cols(const ColArgs& args, int4*, int64_t r, bool) : a(args), row(r)
+    {
+        ld<R>(a.desc + r, ds);
+    }
+    template <int NS>
+    __device__ __forceinline__ void issue(Win<NS>& w, int start) const
+    {
+#pragma unroll
+        for(int q = 0; q < NS; ++q) ld_nt<R>(a.col + ell_at(start + q, row), w.c[q]);
+    }
+    __device__ __forceinline__ void join() {}
+    // neighbour values of every loaded slot that has a column (a slot the row
+    // does not use reads a value that is then ignored: its own diagonal, or a
+    // neighbour outside the window's kind -- never a row this launch writes)
+    template <int NS, typename XT>
+    __device__ __forceinline__ void gather(const Win<NS>& w, int, const XT* __restrict__ x,
+                                           XT (&xv)[slot_dim(NS)][R]) const
+    {
+#pragma unroll
+        for(int q = 0; q < NS; ++q)
+#pragma unroll
+            for(int k = 0; k < R; ++k) xv[q][k] = (w.c[q][k] >= 0) ? x[w.c[q][k]] : (XT)0;
+    }
+};
+
+template <int R, int BS>
+struct Cols<true, R, BS>
+{
+    template <int NS>
+    struct Win
+    {
+    };
+    const int4* tab;
+    int4* lds;        // the colour's patterns, PAT_QUADS int4 each
+    int n;            // int4s of them
+    uint32_t row;
+    bool stage;       // this call loads the patterns (block-uniform)
+    int4 part;        // this thread's first int4 of them, on its way to LDS
+    int id[R];
+    int32_t ds[R];
+    __device__ __forceinline__ Cols(const ColArgs& a, int4* l, int64_t r, bool st)
+        : tab((const int4*)a.tab), lds(l), n(a.npat * PAT_QUADS), row((uint32_t)r), stage(st)
+    {
+        part = tab[min((int)threadIdx.x, n - 1)];
+        if constexpr(R == 1)
+            id[0] = a.pat[r];
+        else
+        {
+            const int w = *reinterpret_cast<const uint16_t*>(a.pat + r);   // r is even
+            id[0] = w & 255;
+            id[1] = w >> 8;
+        }
+    }
+    template <int NS>
+    __device__ __forceinline__ void issue(Win<NS>&, int) const
+    {
+    }
+    // every thread of the block calls this (threads past the end of the rows
+    // work on a row in range and do not store)
+    __device__ __forceinline__ void join()
+    {
+        if(stage)
+        {
+            if((int)threadIdx.x < n) lds[threadIdx.x] = part;
+            for(int k = threadIdx.x + BS; k < n; k += BS) lds[k] = tab[k];
+            __syncthreads();
+        }
+#pragma unroll
+        for(int k = 0; k < R; ++k) ds[k] = lds[id[k] * PAT_QUADS + PAT_QUADS - 1].w;
+    }
+    // unused slots read the row's own x (offset 0); the value is ignored
+    template <int NS, typename XT>
+    __device__ __forceinline__ void gather(const Win<NS>&, int start, const XT* __restrict__ x,
+                                           XT (&xv)[slot_dim(NS)][R]) const
+    {
+#pragma unroll
+        for(int k = 0; k < R; ++k)
+#pragma unroll
+            for(int g = start / 4; g < PAT_QUADS && NS > 0; ++g)
+            {
+                if(4 * g >= start + NS) continue;
+                const int4 o4 = lds[id[k] * PAT_QUADS + g];
+                const int32_t o[4] = {o4.x, o4.y, o4.z, o4.w};
+#pragma unroll
+                for(int j = 0; j < 4; ++j)
+                {
+                    const int q = 4 * g + j - start;
+                    if(q < 0 || q >= NS) continue;
+                    const uint32_t at = (row + (uint32_t)k + (uint32_t)o[j]) * (uint32_t)sizeof(XT);
+                    xv[q][k] = *reinterpret_cast<const XT*>(reinterpret_cast<const char*>(x) + at);
+                }
+            }
+    }
+};
+
+// ---------------------------------------------------------------------------
+// Row bodies shared by the single-problem kernels (ops.hip) and the batched
+// kernels (batch.hip).  A thread owns rows [row, row+R) (R-aligned); with
+// live = false it computes on rows in range and stores nothing.
+
+template <int NS, typename VT, int R>
+__device__ __forceinline__ void load_vals(int64_t row, const VT* __restrict__ val, int start,
+                                          VT (&av)[slot_dim(NS)][R])
 {
 #pragma unroll
-    for(int q = 0; q < NS; ++q)
-#pragma unroll
-        for(int k = 0; k < R; ++k) xv[q][k] = (cc[q][k] >= 0) ? x[cc[q][k]] : (XT)0;
+    for(int q = 0; q < NS; ++q) ld_nt<R>(val + ell_at(start + q, row), av[q]);
 }
 
 // s -= a x over the window's slots in [lo, hi) of each row, ascending.
 template <int NS, typename VT, typename XT, int R>
 __device__ __forceinline__ void sub_window(int start, const int (&lo)[R], const int (&hi)[R],
-                                           const int32_t (&cc)[slot_dim(NS)][R],
                                            const VT (&av)[slot_dim(NS)][R], const XT (&xv)[slot_dim(NS)][R],
                                            XT (&s)[R])
 {
@@ -334,40 +422,61 @@ __device__ __forceinline__ void sub_window(int start, const int (&lo)[R], const 
     for(int q = 0; q < NS; ++q)
 #pragma unroll
         for(int k = 0; k < R; ++k)
-            if(start + q >= lo[k] && start + q < hi[k] && cc[q][k] >= 0)
-                s[k] = fmaT(-cvt<XT>(av[q][k]), xv[q][k], s[k]);
+            if(start + q >= lo[k] && start + q < hi[k]) s[k] = fmaT(-cvt<XT>(av[q][k]), xv[q][k], s[k]);
+}
+
+// y = A x on R rows; returns the row sums in s[].
+template <typename VT, typename XT, int R, typename C>
+__device__ __forceinline__ void row_spmv(int64_t row, C& cols, const VT* __restrict__ val,
+                                         const XT* __restrict__ x, XT (&s)[R])
+{
+    typename C::template Win<W> w;
+    VT av[W][R];
+    cols.template issue<W>(w, 0);
+    load_vals<W, VT, R>(row, val, 0, av);
+    cols.join();
+    XT xv[W][R];
+    cols.template gather<W, XT>(w, 0, x, xv);
+#pragma unroll
+    for(int k = 0; k < R; ++k) s[k] = 0;
+#pragma unroll
+    for(int p = 0; p < W; ++p)
+#pragma unroll
+        for(int k = 0; k < R; ++k)
+            if(p <= desc_diag(cols.ds[k]) || p >= desc_upper(cols.ds[k]))
+                s[k] = fmaT(cvt<XT>(av[p][k]), xv[p][k], s[k]);
 }
 
 // Zero-initial-guess forward sweep: only entries left of the diagonal
 // (earlier colours) are non-zero in x.  Window [0, NS), NS >= the colour's
-// largest d; the diagonal comes from its own array (dg).
-template <int NS, typename VT, typename XT, typename RT, int R>
-__device__ __forceinline__ void row_fwd_zero(int64_t row, const int32_t* __restrict__ col,
-                                             const VT* __restrict__ val, const VT* __restrict__ dg,
-                                             const int32_t* __restrict__ desc, const RT* __restrict__ r,
+// largest d; the diagonal comes from its own array (dg).  A row of the last
+// colour has no upper entries, so this is its full forward sweep too.
+template <int NS, typename VT, typename XT, typename RT, int R, typename C>
+__device__ __forceinline__ void row_fwd_zero(int64_t row, bool live, C& cols, const VT* __restrict__ val,
+                                             const VT* __restrict__ dg, const RT* __restrict__ r,
                                              XT* __restrict__ x)
 {
-    int32_t ds[R];
-    ld<R>(desc + row, ds);
-    int32_t cc[slot_dim(NS)][R];
+    typename C::template Win<NS> w;
     VT av[slot_dim(NS)][R];
-    load_window<NS, VT, R>(row, col, val, 0, cc, av);
+    cols.template issue<NS>(w, 0);
+    load_vals<NS, VT, R>(row, val, 0, av);
     XT d[R], s[R];
     ld_cvt<R>(dg + row, d);
     ld_cvt<R>(r + row, s);
+    cols.join();
     XT xv[slot_dim(NS)][R];
-    gather<NS, XT, R>(cc, x, xv);
+    cols.template gather<NS, XT>(w, 0, x, xv);
     int lo[R], hi[R];
 #pragma unroll
     for(int k = 0; k < R; ++k)
     {
         lo[k] = 0;
-        hi[k] = desc_diag(ds[k]);
+        hi[k] = desc_diag(cols.ds[k]);
     }
-    sub_window<NS, VT, XT, R>(0, lo, hi, cc, av, xv, s);
+    sub_window<NS, VT, XT, R>(0, lo, hi, av, xv, s);
 #pragma unroll
     for(int k = 0; k < R; ++k) s[k] = s[k] / d[k];
-    st<R>(x + row, s);
+    if(live) st<R>(x + row, s);
 }
 
 // Zero-initial-guess backward sweep: x = (x*d - U x) / d over the upper
@@ -377,35 +486,33 @@ __device__ __forceinline__ void row_fwd_zero(int64_t row, const int32_t* __restr
 // for the post-smoother's forward sweep (row_fwd_full_u); u is read off the
 // running sum (x*d minus its value on reaching slot tl), so it costs no second
 // accumulation.
-template <int NS, typename VT, typename XT, bool STORE_U, int R>
-__device__ __forceinline__ void row_bwd_zero(int64_t row, const int32_t* __restrict__ col,
-                                             const VT* __restrict__ val, const VT* __restrict__ dg,
-                                             const int32_t* __restrict__ desc, XT* __restrict__ x,
-                                             XT* __restrict__ u)
+template <int NS, typename VT, typename XT, bool STORE_U, int R, typename C>
+__device__ __forceinline__ void row_bwd_zero(int64_t row, bool live, C& cols, const VT* __restrict__ val,
+                                             const VT* __restrict__ dg, XT* __restrict__ x, XT* __restrict__ u)
 {
     // u = x*d - snap must use the rounded product that starts the running
     // sum: left to the compiler, the product may or may not be contracted
     // into the subtraction depending on the instruction schedule, and then
     // two launch shapes of the same operator round u differently.
 #pragma clang fp contract(off)
-    int32_t ds[R];
-    ld<R>(desc + row, ds);
     const int start = W - NS;
-    int32_t cc[slot_dim(NS)][R];
+    typename C::template Win<NS> w;
     VT av[slot_dim(NS)][R];
-    load_window<NS, VT, R>(row, col, val, start, cc, av);
+    cols.template issue<NS>(w, start);
+    load_vals<NS, VT, R>(row, val, start, av);
     XT d[R], s[R];
     ld_cvt<R>(dg + row, d);
     ld<R>(x + row, s);
 #pragma unroll
     for(int k = 0; k < R; ++k) s[k] = s[k] * d[k];
+    cols.join();
     XT xv[slot_dim(NS)][R];
-    gather<NS, XT, R>(cc, x, xv);
+    cols.template gather<NS, XT>(w, start, x, xv);
     int lo[R], hi[R];
 #pragma unroll
     for(int k = 0; k < R; ++k)
     {
-        lo[k] = desc_upper(ds[k]);
+        lo[k] = desc_upper(cols.ds[k]);
         hi[k] = W;
     }
     if constexpr(STORE_U)
@@ -426,49 +533,43 @@ __device__ __forceinline__ void row_bwd_zero(int64_t row, const int32_t* __restr
 #pragma unroll
             for(int k = 0; k < R; ++k)
             {
-                if(!taken[k] && start + q >= desc_tail(ds[k]))
+                if(!taken[k] && start + q >= desc_tail(cols.ds[k]))
                 {
                     snap[k] = s[k];
                     taken[k] = true;
                 }
-                if(start + q >= lo[k] && cc[q][k] >= 0) s[k] = fmaT(-cvt<XT>(av[q][k]), xv[q][k], s[k]);
+                if(start + q >= lo[k]) s[k] = fmaT(-cvt<XT>(av[q][k]), xv[q][k], s[k]);
             }
         XT uu[R];
 #pragma unroll
         for(int k = 0; k < R; ++k) uu[k] = s0[k] - (taken[k] ? snap[k] : s[k]);
-        st<R>(u + row, uu);
+        if(live) st<R>(u + row, uu);
     }
     else
     {
-        sub_window<NS, VT, XT, R>(start, lo, hi, cc, av, xv, s);
+        sub_window<NS, VT, XT, R>(start, lo, hi, av, xv, s);
     }
 #pragma unroll
     for(int k = 0; k < R; ++k) s[k] = s[k] / d[k];
-    st<R>(x + row, s);
+    if(live) st<R>(x + row, s);
 }
 
 // Full forward sweep over the whole row in ascending column order; keeps
 // t = r - L x (the sum up to the diagonal) for the backward sweep, whose lower
 // neighbours do not change in between.
-template <typename VT, typename XT, typename RT, bool STORE_T, int R>
-__device__ __forceinline__ void row_fwd_full(int64_t row, const int32_t* __restrict__ col,
-                                             const VT* __restrict__ val, const RT* __restrict__ r,
-                                             XT* __restrict__ x, XT* __restrict__ t)
+template <typename VT, typename XT, typename RT, int R, typename C>
+__device__ __forceinline__ void row_fwd_full(int64_t row, bool live, C& cols, const VT* __restrict__ val,
+                                             const RT* __restrict__ r, XT* __restrict__ x, XT* __restrict__ t)
 {
-    int32_t cc[W][R];
+    typename C::template Win<W> w;
     VT av[W][R];
-#pragma unroll
-    for(int p = 0; p < W; ++p) ld_nt<R>(col + ell_at(p, row), cc[p]);
-#pragma unroll
-    for(int p = 0; p < W; ++p) ld_nt<R>(val + ell_at(p, row), av[p]);
-    XT xv[W][R];
-#pragma unroll
-    for(int p = 0; p < W; ++p)
-#pragma unroll
-        for(int k = 0; k < R; ++k)
-            xv[p][k] = (cc[p][k] >= 0 && (int64_t)cc[p][k] != row + k) ? x[cc[p][k]] : (XT)0;
+    cols.template issue<W>(w, 0);
+    load_vals<W, VT, R>(row, val, 0, av);
     XT s[R], tt[R], d[R];
     ld_cvt<R>(r + row, s);
+    cols.join();
+    XT xv[W][R];
+    cols.template gather<W, XT>(w, 0, x, xv);
 #pragma unroll
     for(int k = 0; k < R; ++k)
     {
@@ -480,23 +581,19 @@ __device__ __forceinline__ void row_fwd_full(int64_t row, const int32_t* __restr
 #pragma unroll
         for(int k = 0; k < R; ++k)
         {
-            if(cc[p][k] >= 0)
+            const int dk = desc_diag(cols.ds[k]);
+            if(p == dk)
             {
-                if((int64_t)cc[p][k] == row + k)
-                {
-                    tt[k] = s[k];
-                    d[k] = cvt<XT>(av[p][k]);
-                }
-                else
-                {
-                    s[k] = fmaT(-cvt<XT>(av[p][k]), xv[p][k], s[k]);
-                }
+                tt[k] = s[k];
+                d[k] = cvt<XT>(av[p][k]);
             }
+            else if(p < dk || p >= desc_upper(cols.ds[k]))
+                s[k] = fmaT(-cvt<XT>(av[p][k]), xv[p][k], s[k]);
         }
 #pragma unroll
     for(int k = 0; k < R; ++k) s[k] = s[k] / d[k];
-    st<R>(x + row, s);
-    if(STORE_T) st<R>(t + row, tt);
+    if(live) st<R>(x + row, s);
+    if(live) st<R>(t + row, tt);
 }
 
 // The post-smoother's forward sweep for a row of a colour before the last,
@@ -506,36 +603,37 @@ __device__ __forceinline__ void row_fwd_full(int64_t row, const int32_t* __restr
 // last-colour entries [tl, W) at their corrected x.  Reads the lower, the
 // diagonal and the last-colour slots only: windows [0, NA) and [W - NB, W);
 // t[row] becomes r - L x.
-template <int NA, int NB, typename VT, typename XT, typename RT, int R>
-__device__ __forceinline__ void row_fwd_full_u(int64_t row, const int32_t* __restrict__ col,
-                                               const VT* __restrict__ val,
-                                               const VT* __restrict__ dg, const int32_t* __restrict__ desc,
-                                               const RT* __restrict__ r, XT* __restrict__ x, XT* __restrict__ t)
+template <int NA, int NB, typename VT, typename XT, typename RT, int R, typename C>
+__device__ __forceinline__ void row_fwd_full_u(int64_t row, bool live, C& cols, const VT* __restrict__ val,
+                                               const VT* __restrict__ dg, const RT* __restrict__ r,
+                                               XT* __restrict__ x, XT* __restrict__ t)
 {
-    int32_t ds[R];
-    ld<R>(desc + row, ds);
     const int bstart = W - NB;
-    int32_t ca[slot_dim(NA)][R], cb[slot_dim(NB)][R];
+    typename C::template Win<NA> wa;
+    typename C::template Win<NB> wb;
     VT aa[slot_dim(NA)][R], ab[slot_dim(NB)][R];
-    load_window<NA, VT, R>(row, col, val, 0, ca, aa);
-    load_window<NB, VT, R>(row, col, val, bstart, cb, ab);
+    cols.template issue<NA>(wa, 0);
+    load_vals<NA, VT, R>(row, val, 0, aa);
+    cols.template issue<NB>(wb, bstart);
+    load_vals<NB, VT, R>(row, val, bstart, ab);
     XT d[R], s[R], uu[R];
     ld_cvt<R>(dg + row, d);
     ld_cvt<R>(r + row, s);
     ld<R>(t + row, uu);
+    cols.join();
     XT xa[slot_dim(NA)][R], xb[slot_dim(NB)][R];
-    gather<NA, XT, R>(ca, x, xa);
-    gather<NB, XT, R>(cb, x, xb);
+    cols.template gather<NA, XT>(wa, 0, x, xa);
+    cols.template gather<NB, XT>(wb, bstart, x, xb);
     int alo[R], ahi[R], blo[R], bhi[R];
 #pragma unroll
     for(int k = 0; k < R; ++k)
     {
         alo[k] = 0;
-        ahi[k] = desc_diag(ds[k]);
-        blo[k] = desc_tail(ds[k]);
+        ahi[k] = desc_diag(cols.ds[k]);
+        blo[k] = desc_tail(cols.ds[k]);
         bhi[k] = W;
     }
-    sub_window<NA, VT, XT, R>(0, alo, ahi, ca, aa, xa, s);
+    sub_window<NA, VT, XT, R>(0, alo, ahi, aa, xa, s);
     XT tt[R];
 #pragma unroll
     for(int k = 0; k < R; ++k)
@@ -543,68 +641,62 @@ __device__ __forceinline__ void row_fwd_full_u(int64_t row, const int32_t* __res
         tt[k] = s[k];
         s[k] = s[k] - uu[k];
     }
-    sub_window<NB, VT, XT, R>(bstart, blo, bhi, cb, ab, xb, s);
+    sub_window<NB, VT, XT, R>(bstart, blo, bhi, ab, xb, s);
 #pragma unroll
     for(int k = 0; k < R; ++k) s[k] = s[k] / d[k];
-    st<R>(x + row, s);
-    st<R>(t + row, tt);
+    if(live) st<R>(x + row, s);
+    if(live) st<R>(t + row, tt);
 }
 
 // Full backward sweep from t: x = (t - U x) / d over the upper entries,
 // window [W - NS, W).
-template <int NS, typename VT, typename XT, int R>
-__device__ __forceinline__ void row_bwd_full(int64_t row, const int32_t* __restrict__ col,
-                                             const VT* __restrict__ val, const VT* __restrict__ dg,
-                                             const int32_t* __restrict__ desc, const XT* __restrict__ t,
+template <int NS, typename VT, typename XT, int R, typename C>
+__device__ __forceinline__ void row_bwd_full(int64_t row, bool live, C& cols, const VT* __restrict__ val,
+                                             const VT* __restrict__ dg, const XT* __restrict__ t,
                                              XT* __restrict__ x)
 {
-    int32_t ds[R];
-    ld<R>(desc + row, ds);
     const int start = W - NS;
-    int32_t cc[slot_dim(NS)][R];
+    typename C::template Win<NS> w;
     VT av[slot_dim(NS)][R];
-    load_window<NS, VT, R>(row, col, val, start, cc, av);
+    cols.template issue<NS>(w, start);
+    load_vals<NS, VT, R>(row, val, start, av);
     XT d[R], s[R];
     ld_cvt<R>(dg + row, d);
     ld<R>(t + row, s);
+    cols.join();
     XT xv[slot_dim(NS)][R];
-    gather<NS, XT, R>(cc, x, xv);
+    cols.template gather<NS, XT>(w, start, x, xv);
     int lo[R], hi[R];
 #pragma unroll
     for(int k = 0; k < R; ++k)
     {
-        lo[k] = desc_upper(ds[k]);
+        lo[k] = desc_upper(cols.ds[k]);
         hi[k] = W;
     }
-    sub_window<NS, VT, XT, R>(start, lo, hi, cc, av, xv, s);
+    sub_window<NS, VT, XT, R>(start, lo, hi, av, xv, s);
 #pragma unroll
     for(int k = 0; k < R; ++k) s[k] = s[k] / d[k];
-    st<R>(x + row, s);
+    if(live) st<R>(x + row, s);
 }
 
-// Fused fine residual + injection for coarse natural row k:
-// rc[f2c_coarse[k]] = r[f] - sum_p a[f,p] x[col], f = f2c_fine[k].
-template <typename VT, typename XT, typename RT, typename CT>
-__device__ __forceinline__ void row_restrict(int64_t k, const int32_t* __restrict__ col,
-                                             const VT* __restrict__ val, const int32_t* __restrict__ f2c_fine,
-                                             const int32_t* __restrict__ f2c_coarse, const RT* __restrict__ r,
-                                             const XT* __restrict__ x, CT* __restrict__ rc)
+// Fused fine residual + injection for the coarse row at fine row `row`:
+// returns r - sum_p a[p] x[col].
+template <typename VT, typename XT, typename RT, typename C>
+__device__ __forceinline__ XT row_restrict(int64_t row, C& cols, const VT* __restrict__ val,
+                                           const RT* __restrict__ r, const XT* __restrict__ x)
 {
-    const int64_t row = f2c_fine[k];
-    int32_t cc[W][1];
+    typename C::template Win<W> w;
     VT av[W][1];
-#pragma unroll
-    for(int p = 0; p < W; ++p) ld_nt<1>(col + ell_at(p, row), cc[p]);
-#pragma unroll
-    for(int p = 0; p < W; ++p) ld_nt<1>(val + ell_at(p, row), av[p]);
-    XT xv[W];
-#pragma unroll
-    for(int p = 0; p < W; ++p) xv[p] = (cc[p][0] >= 0) ? x[cc[p][0]] : (XT)0;
+    cols.template issue<W>(w, 0);
+    load_vals<W, VT, 1>(row, val, 0, av);
     XT s = cvt<XT>(r[row]);
+    cols.join();
+    XT xv[W][1];
+    cols.template gather<W, XT>(w, 0, x, xv);
 #pragma unroll
     for(int p = 0; p < W; ++p)
-        if(cc[p][0] >= 0) s = fmaT(-cvt<XT>(av[p][0]), xv[p], s);
-    rc[f2c_coarse[k]] = (CT)s;
+        if(p <= desc_diag(cols.ds[0]) || p >= desc_upper(cols.ds[0])) s = fmaT(-cvt<XT>(av[p][0]), xv[p][0], s);
+    return s;
 }
 
 // ---------------------------------------------------------------------------

@@ -1,4 +1,5 @@
-// ops.hip -- the solver's hot-path kernels for gfx950 (CDNA4, wave64).
+// ops.hip -- the solver's hot-path kernels for gfx950 (CDNA4, wave64), but for
+// the SymGS sweeps (sweeps.hpp).
 //
 // All operators are HBM-bound sparse/streaming work: one thread per row,
 // sliced ELL (entry p of row r at ell_at(p, r), common.hpp) so every slot load
@@ -9,15 +10,13 @@
 //
 // Reference kernels whose results these reproduce:
 //   SpMV                kernel_spmv_ell           ComputeSPMV.cpp:130-170
-//   SymGS sweep         kernel_symgs_sweep        ComputeSYMGS.cpp:113-151, :369-404
-//   zero-guess SymGS    kernel_pointwise_mult / kernel_forward_sweep_0 /
-//                       kernel_backward_sweep_0   ComputeSYMGS.cpp:238-341, :406-454
 //   residual+restrict   kernel_fused_restrict_spmv ComputeRestriction.cpp:81-124
 //   prolongation        kernel_prolongation       ComputeProlongation.cpp:39-59
 //   dot / waxpby / fused waxpby-dot               ComputeDotProduct.cpp:63-238,
 //                                                 ComputeWAXPBY.cpp:63-240
 #include "common.hpp"
 #include "kernels.hpp"
+#include "launch.hpp"
 #include "ops.hpp"
 
 #include <algorithm>
@@ -26,12 +25,12 @@
 namespace hpcgx
 {
 
-template <typename VT, typename XT, typename YT, bool DOT, int R, int BS>
-__global__ __launch_bounds__(BS) void k_spmv(const int32_t* __restrict__ col,
-                                            const VT* __restrict__ val, const XT* __restrict__ x,
+template <bool PAT, typename VT, typename XT, typename YT, bool DOT, int R, int BS>
+__global__ __launch_bounds__(BS) void k_spmv(ColArgs ca, const VT* __restrict__ val, const XT* __restrict__ x,
                                             YT* __restrict__ y, Tiles tl, RedArgs ra, const int* gate)
 {
     if(gated(gate)) return;
+    PAT_LDS();
     const int64_t ntiles = (int64_t)tl.ncolors * tl.jtiles;
     const int64_t L = xcd_block(blockIdx.x, gridDim.x);
     const int64_t g0 = (L / tl.gx) * tl.gx;   // first block of L's group
@@ -40,14 +39,23 @@ __global__ __launch_bounds__(BS) void k_spmv(const int32_t* __restrict__ col,
     const int64_t t0 = g0 * tl.tpb + (L - g0);
     const int64_t t1 = e < ntiles ? e : ntiles;
     double acc = 0.0;
+    int staged = -1;   // colour whose patterns are in LDS
     for(int64_t t = t0; t < t1; t += members)
     {
         const int c = (int)(t % tl.ncolors);
-        const int64_t i = (t / tl.ncolors) * (BS * R) + (int64_t)threadIdx.x * R;
-        if(i >= tl.size[c]) continue;
-        const int64_t row = tl.off[c] + i;
+        const int64_t i0 = (t / tl.ncolors) * (BS * R);
+        if(i0 >= tl.size[c]) continue;   // uniform over the block
+        const int64_t i = i0 + (int64_t)threadIdx.x * R;
+        const bool live = i < tl.size[c];
+        const int64_t row = tl.off[c] + (live ? i : tl.size[c] - R);
+        if(PAT && staged >= 0 && staged != c) __syncthreads();   // the other waves are done with the old ones
+        ColArgs cc = ca;
+        cc.tab = ca.tab + (int64_t)c * (PAT_MAX * PAT_QUADS * 4);
+        Cols<PAT, R, BS> cols(cc, pat_lds, row, staged != c);
+        staged = c;
         XT s[R];
-        row_spmv<VT, XT, R>(row, col, val, x, s);
+        row_spmv<VT, XT, R>(row, cols, val, x, s);
+        if(!live) continue;
         st_cvt<R>(y + row, s);
         if(DOT)
         {
@@ -60,88 +68,22 @@ __global__ __launch_bounds__(BS) void k_spmv(const int32_t* __restrict__ col,
     if(DOT) block_partial<BS>(acc, ra.partial, blockIdx.x);
 }
 
-// Per-colour sweeps: block b covers rows off + T*BS*R + [0, BS*R), where T is
-// L = xcd_block(b), mapped through the colour's column order (ZMap) on large
-// planes.  Consecutive colour launches alternate direction (size < 0 marks a
-// reversed launch): each XCD then starts a launch on the slab it finished the
-// previous one on, whose neighbours' x is still in its caches.
-#define SWEEP_ROW()                                                                   \
-    if(gated(gate)) return;                                                           \
-    int64_t Lb_ = xcd_block(blockIdx.x, gridDim.x);                                   \
-    if(size < 0)                                                                      \
-    {                                                                                 \
-        size = -size;                                                                 \
-        Lb_ = (int64_t)gridDim.x - 1 - Lb_;                                           \
-    }                                                                                 \
-    if(zm.k > 1)                                                                      \
-    {                                                                                 \
-        const unsigned per_ = (unsigned)zm.planes * (unsigned)zm.tpc;                 \
-        const unsigned lb_ = (unsigned)Lb_, col_ = lb_ / per_, rem_ = lb_ - col_ * per_; \
-        const unsigned pl_ = rem_ / (unsigned)zm.tpc;                                 \
-        Lb_ = ((int64_t)pl_ * zm.k + col_) * zm.tpc + (rem_ - pl_ * (unsigned)zm.tpc); \
-    }                                                                                 \
-    const int64_t i = Lb_ * (BS * R) + (int64_t)threadIdx.x * R;                      \
-    if(i >= size) return;                                                             \
-    const int64_t row = off + i;
-
-template <int NS, typename VT, typename XT, typename RT, int R, int BS>
-__global__ __launch_bounds__(BS) void k_fwd_zero(int64_t off, int64_t size, ZMap zm, const int32_t* __restrict__ col, const VT* __restrict__ val,
-                                                 const VT* __restrict__ dg, const int32_t* __restrict__ desc,
-                                                 const RT* __restrict__ r, XT* __restrict__ x, const int* gate)
-{
-    SWEEP_ROW();
-    row_fwd_zero<NS, VT, XT, RT, R>(row, col, val, dg, desc, r, x);
-}
-
-template <int NS, typename VT, typename XT, bool STORE_U, int R, int BS>
-__global__ __launch_bounds__(BS) void k_bwd_zero(int64_t off, int64_t size, ZMap zm, const int32_t* __restrict__ col, const VT* __restrict__ val,
-                                                 const VT* __restrict__ dg, const int32_t* __restrict__ desc,
-                                                 XT* __restrict__ x, XT* __restrict__ u, const int* gate)
-{
-    SWEEP_ROW();
-    row_bwd_zero<NS, VT, XT, STORE_U, R>(row, col, val, dg, desc, x, u);
-}
-
-template <typename VT, typename XT, typename RT, bool STORE_T, int R, int BS>
-__global__ __launch_bounds__(BS) void k_fwd_full(int64_t off, int64_t size, ZMap zm, const int32_t* __restrict__ col,
-                                                 const VT* __restrict__ val, const RT* __restrict__ r,
-                                                 XT* __restrict__ x, XT* __restrict__ t, const int* gate)
-{
-    SWEEP_ROW();
-    row_fwd_full<VT, XT, RT, STORE_T, R>(row, col, val, r, x, t);
-}
-
-template <int NA, int NB, typename VT, typename XT, typename RT, int R, int BS>
-__global__ __launch_bounds__(BS) void k_fwd_full_u(int64_t off, int64_t size, ZMap zm,
-                                                   const int32_t* __restrict__ col, const VT* __restrict__ val,
-                                                   const VT* __restrict__ dg, const int32_t* __restrict__ desc,
-                                                   const RT* __restrict__ r, XT* __restrict__ x, XT* __restrict__ t,
-                                                   const int* gate)
-{
-    SWEEP_ROW();
-    row_fwd_full_u<NA, NB, VT, XT, RT, R>(row, col, val, dg, desc, r, x, t);
-}
-
-template <int NS, typename VT, typename XT, int R, int BS>
-__global__ __launch_bounds__(BS) void k_bwd_full(int64_t off, int64_t size, ZMap zm, const int32_t* __restrict__ col, const VT* __restrict__ val,
-                                                 const VT* __restrict__ dg, const int32_t* __restrict__ desc,
-                                                 const XT* __restrict__ t, XT* __restrict__ x, const int* gate)
-{
-    SWEEP_ROW();
-    row_bwd_full<NS, VT, XT, R>(row, col, val, dg, desc, t, x);
-}
-#undef SWEEP_ROW
-
-template <typename VT, typename XT, typename RT, typename CT, int BS>
-__global__ __launch_bounds__(BS) void k_restrict(int64_t mc, const int32_t* __restrict__ col,
-                                                 const VT* __restrict__ val, const int32_t* __restrict__ f2c_fine,
+// Fused fine residual + injection: rc[f2c_coarse[k]] = (r - A x)[f2c_fine[k]].
+// PAT: every injected row is in the last colour, whose patterns `ca` holds.
+template <bool PAT, typename VT, typename XT, typename RT, typename CT, int BS>
+__global__ __launch_bounds__(BS) void k_restrict(int64_t mc, ColArgs ca, const VT* __restrict__ val,
+                                                 const int32_t* __restrict__ f2c_fine,
                                                  const int32_t* __restrict__ f2c_coarse, const RT* __restrict__ r,
                                                  const XT* __restrict__ x, CT* __restrict__ rc, const int* gate)
 {
     if(gated(gate)) return;
+    PAT_LDS();
     const int64_t k = xcd_block(blockIdx.x, gridDim.x) * BS + threadIdx.x;
-    if(k >= mc) return;
-    row_restrict<VT, XT, RT, CT>(k, col, val, f2c_fine, f2c_coarse, r, x, rc);
+    const int64_t kk = k < mc ? k : mc - 1;
+    const int64_t row = f2c_fine[kk];
+    Cols<PAT, 1, BS> cols(ca, pat_lds, row, true);
+    const XT s = row_restrict<VT, XT, RT>(row, cols, val, r, x);
+    if(k < mc) rc[f2c_coarse[k]] = (CT)s;
 }
 
 // Prolongation: xf[f2c_fine[k]] += xc[f2c_coarse[k]].
@@ -409,10 +351,6 @@ __global__ void k_testcg_scale(int64_t m, double* __restrict__ d, double* __rest
 
 // ---------------------------------------------------------------------------
 // host launchers
-static inline unsigned nblk(int64_t n, int bs) { return (unsigned)ceil_div(n, bs); }
-
-#define HPCGX_KCHECK() HPCGX_HIP(hipGetLastError())
-
 // the fold that completes a reduction whose producer ran `nparts` blocks
 int launch_fold(int64_t nparts, const RedArgs& ra, hipStream_t s, const int* gate)
 {
@@ -421,38 +359,9 @@ int launch_fold(int64_t nparts, const RedArgs& ra, hipStream_t s, const int* gat
     return 0;
 }
 
-// Launch shapes compiled in: rows per thread {1,2} x block {64,128,256}.
-template <typename F>
-static int with_shape(const Shape& sh, F&& f)
-{
-    using std::integral_constant;
-    switch(sh.rows * 1000 + sh.block)
-    {
-    case 1064: return f(integral_constant<int, 1>{}, integral_constant<int, 64>{});
-    case 1128: return f(integral_constant<int, 1>{}, integral_constant<int, 128>{});
-    case 1256: return f(integral_constant<int, 1>{}, integral_constant<int, 256>{});
-    case 2064: return f(integral_constant<int, 2>{}, integral_constant<int, 64>{});
-    case 2128: return f(integral_constant<int, 2>{}, integral_constant<int, 128>{});
-    case 2256: return f(integral_constant<int, 2>{}, integral_constant<int, 256>{});
-    default: break;
-    }
-    set_error("unsupported launch shape (rows " + std::to_string(sh.rows) + ", block " + std::to_string(sh.block) + ")");
-    return -2;
-}
-
 bool shape_supported(int rows, int block)
 {
     return (rows == 1 || rows == 2) && (block == 64 || block == 128 || block == 256);
-}
-
-// R rows per thread need every colour block to be R-aligned (a thread's R
-// rows then share their ELL slice).
-static Shape fit(const Level& L, Shape sh)
-{
-    bool ok = true;
-    for(int c = 0; c < L.ncolors && ok; ++c) ok = (L.offsets[c] % sh.rows) == 0 && (L.sizes[c] % sh.rows) == 0;
-    if(!ok) sh.rows = 1;
-    return sh;
 }
 
 // With a fused dot, a block walks tpb tiles so that the partials stay few
@@ -476,6 +385,9 @@ static Tiles make_tiles(const Level& L, int rows_per_tile, bool dot, int64_t res
     while(dot && ceil_div(ntiles, t.tpb) > cap) ++t.tpb;
     nblocks = ceil_div(ntiles, t.tpb);
     t.gx = (int)std::max<int64_t>(1, resident / NUM_XCD);
+    // a whole number of colours: a block then stays on one colour and stages
+    // its patterns once
+    if(t.gx > t.ncolors) t.gx -= t.gx % t.ncolors;
     return t;
 }
 
@@ -495,44 +407,32 @@ static int64_t resident_blocks(K kernel, int bs, int64_t& cache)
     return cache;
 }
 
-// element-type views of a level's arrays
-template <typename VT>
-static const VT* vals_of(const Level& L);
-template <>
-const double* vals_of<double>(const Level& L) { return L.ell_val; }
-template <>
-const __half* vals_of<__half>(const Level& L) { return L.ell_h; }
-
-template <typename VT>
-static const VT* diag_of(const Level& L);
-template <>
-const double* diag_of<double>(const Level& L) { return L.diag64; }
-template <>
-const __half* diag_of<__half>(const Level& L) { return L.diag_h; }
-
 template <typename VT, typename XT, typename YT>
 static int spmv_t(const Level& L, const void* x, void* y, const RedArgs* ra, hipStream_t s, const int* gate)
 {
     const Shape sh = fit(L, L.shp[std::is_same<VT, double>::value ? PREC_F64 : PREC_MIXED][SH_SPMV]);
     return with_shape(sh, [&](auto RR, auto BB) -> int {
         constexpr int R = decltype(RR)::value, BS = decltype(BB)::value;
-        int64_t nb;
-        if(ra)
-        {
-            const int64_t cap = std::min<int64_t>(ra->cap, FOLD_MAX);
-            static int64_t resident = 0;
-            Tiles tl = make_tiles(L, BS * R, true, resident_blocks(k_spmv<VT, XT, YT, true, R, BS>, BS, resident),
-                                  cap, nb);
-            hipLaunchKernelGGL((k_spmv<VT, XT, YT, true, R, BS>), dim3((unsigned)nb), dim3(BS), 0, s, L.ell_col,
-                               vals_of<VT>(L), (const XT*)x, (YT*)y, tl, *ra, gate);
+        return with_pat(L, [&](auto PP) -> int {
+            constexpr bool PAT = decltype(PP)::value;
+            int64_t nb;
+            if(ra)
+            {
+                const int64_t cap = std::min<int64_t>(ra->cap, FOLD_MAX);
+                static int64_t resident = 0;
+                Tiles tl = make_tiles(L, BS * R, true,
+                                      resident_blocks(k_spmv<PAT, VT, XT, YT, true, R, BS>, BS, resident), cap, nb);
+                hipLaunchKernelGGL((k_spmv<PAT, VT, XT, YT, true, R, BS>), dim3((unsigned)nb), dim3(BS), 0, s,
+                                   L.cols(0), vals_of<VT>(L), (const XT*)x, (YT*)y, tl, *ra, gate);
+                HPCGX_KCHECK();
+                return launch_fold(nb, *ra, s, gate);
+            }
+            Tiles tl = make_tiles(L, BS * R, false, 0, 0, nb);
+            hipLaunchKernelGGL((k_spmv<PAT, VT, XT, YT, false, R, BS>), dim3((unsigned)nb), dim3(BS), 0, s, L.cols(0),
+                               vals_of<VT>(L), (const XT*)x, (YT*)y, tl, RedArgs{}, gate);
             HPCGX_KCHECK();
-            return launch_fold(nb, *ra, s, gate);
-        }
-        Tiles tl = make_tiles(L, BS * R, false, 0, 0, nb);
-        hipLaunchKernelGGL((k_spmv<VT, XT, YT, false, R, BS>), dim3((unsigned)nb), dim3(BS), 0, s, L.ell_col,
-                           vals_of<VT>(L), (const XT*)x, (YT*)y, tl, RedArgs{}, gate);
-        HPCGX_KCHECK();
-        return 0;
+            return 0;
+        });
     });
 }
 
@@ -548,141 +448,6 @@ int launch_spmv_f64x(const Level& L, Prec prec, const double* x, double* y, cons
     // f64 vectors over either value store (f16 values are exact: 26 / -1)
     if(prec == PREC_F64) return spmv_t<double, double, double>(L, x, y, ra, s, gate);
     return spmv_t<__half, double, double>(L, x, y, ra, s, gate);
-}
-
-// The sweeps' block order for a colour of `size` rows in tiles of `tile` rows
-// (grid = its tile count).  Planes of the half-resolution colour grid whose x
-// gathers (7 other colours, 3 planes, 8 B) outgrow an XCD's 4 MB L2 are cut
-// into columns of >= min_rows rows (measured best: 8192 for the f64 sweeps,
-// 4096 for the f16/f32 ones), so that the blocks in flight on an XCD march
-// through one column's planes; Level::zcols > 0 forces a column count.
-static ZMap zmap_for(const Level& L, int64_t size, int tile, unsigned grid, int64_t min_rows)
-{
-    ZMap z;
-    if(L.zcols == 1 || L.ncolors != 8 || ((L.nx | L.ny | L.nz) & 1) != 0) return z;
-    const int64_t plane = (int64_t)(L.nx / 2) * (L.ny / 2), planes = L.nz / 2;
-    if(size != plane * planes || plane % tile) return z;
-    const int64_t tpp = plane / tile;
-    int64_t k = L.zcols;
-    if(k == 0)
-    {
-        if(plane * 8 * 21 <= ((int64_t)6 << 20)) return z;
-        k = 1;
-        while(tpp % (2 * k) == 0 && (tpp / (2 * k)) * tile >= min_rows) k *= 2;
-    }
-    if(k <= 1 || tpp % k || (int64_t)grid != planes * tpp) return z;
-    z.k = (int)k;
-    z.tpc = (int)(tpp / k);
-    z.planes = (int)planes;
-    return z;
-}
-
-// one launch per colour c in [c0, c1) (step +1) or (c0, c1] (step -1); a
-// colour whose slot window (kind `wk`, one row per thread) exceeds 16 slots
-// runs with the op's wide shape, the others with its narrow shape
-template <typename Launch>
-static int per_color(const Level& L, int prec, int which, int wk, int c_first, int c_last, int step,
-                     Launch&& launch)
-{
-    for(int c = c_first; step > 0 ? c <= c_last : c >= c_last; c += step)
-    {
-        if(L.sizes[c] == 0) continue;
-        const bool wide = (wk < 0) || L.win[wk][c] > 16;
-        const Shape sh = fit(L, L.shp[prec][wide ? which : which + SH_NARROW]);
-        HPCGX_TRY(with_shape(sh, [&](auto RR, auto BB) -> int {
-            constexpr int R = decltype(RR)::value, BS = decltype(BB)::value;
-            const dim3 grid(nblk(ceil_div(L.sizes[c], R), BS));
-            // odd colours walk their blocks backwards (in both sweeps: forward
-            // ends on colour 7 reversed, backward starts on colour 6 forwards,
-            // so every launch starts on the slab the previous one ended on)
-            const int64_t size = (c & 1) ? -(int64_t)L.sizes[c] : (int64_t)L.sizes[c];
-            launch(RR, BB, grid, c, size, zmap_for(L, L.sizes[c], BS * R, grid.x, prec == PREC_F64 ? 8192 : 4096));
-            HPCGX_KCHECK();
-            return 0;
-        }));
-    }
-    return 0;
-}
-
-// The sweep kernels of a level: part 0 = zero-guess forward (colours 0..n-1),
-// 1 = zero-guess backward (n-2..0), 2 = forward keeping t (0..n-1), 3 =
-// backward from t (n-2..0), 4 = part 1 also keeping the upper sums outside
-// the last colour in t, 5 = part 2 reusing them (valid after part 4 when
-// only last-colour rows changed in between).
-template <typename VT, typename XT, typename RT>
-static int sweep_t(const Level& L, int part, const void* rv, void* xv, void* tv, hipStream_t s, const int* gate)
-{
-    const RT* r = (const RT*)rv;
-    XT* x = (XT*)xv;
-    XT* t = (XT*)tv;
-    const VT* val = vals_of<VT>(L);
-    const VT* dg = diag_of<VT>(L);
-    const int last = L.ncolors - 1;
-    const int pr = std::is_same<VT, double>::value ? PREC_F64 : PREC_MIXED;
-    using std::integral_constant;
-    switch(part)
-    {
-    case 0:
-        return per_color(L, pr, SH_FWD_ZERO, WIN_LOWER, 0, last, 1, [&](auto RR, auto BB, dim3 grid, int c, int64_t sz, ZMap zm) {
-            constexpr int R = decltype(RR)::value, BS = decltype(BB)::value;
-            const int n = L.win[WIN_LOWER][c];
-            with_window(n, [&](auto NN) {
-                constexpr int NS = decltype(NN)::value;
-                hipLaunchKernelGGL((k_fwd_zero<NS, VT, XT, RT, R, BS>), grid, dim3(BS), 0, s,
-                                   (int64_t)L.offsets[c], sz, zm, L.ell_col, val, dg, L.desc, r, x, gate);
-            });
-        });
-    case 1:
-    case 4:
-        if(last < 1) return 0;
-        return per_color(L, pr, SH_BWD_ZERO, WIN_UPPER, last - 1, 0, -1, [&](auto RR, auto BB, dim3 grid, int c, int64_t sz, ZMap zm) {
-            constexpr int R = decltype(RR)::value, BS = decltype(BB)::value;
-            const int n = L.win[WIN_UPPER][c];
-            with_window(n, [&](auto NN) {
-                constexpr int NS = decltype(NN)::value;
-                if(part == 4)
-                    hipLaunchKernelGGL((k_bwd_zero<NS, VT, XT, true, R, BS>), grid, dim3(BS), 0, s,
-                                       (int64_t)L.offsets[c], sz, zm, L.ell_col, val, dg, L.desc, x, t, gate);
-                else
-                    hipLaunchKernelGGL((k_bwd_zero<NS, VT, XT, false, R, BS>), grid, dim3(BS), 0, s,
-                                       (int64_t)L.offsets[c], sz, zm, L.ell_col, val, dg, L.desc, x, t, gate);
-            });
-        });
-    case 2:
-    case 5:
-        return per_color(L, pr, SH_FWD_FULL, part == 5 ? WIN_LOWER : -1, 0, last, 1, [&](auto RR, auto BB, dim3 grid, int c, int64_t sz, ZMap zm) {
-            constexpr int R = decltype(RR)::value, BS = decltype(BB)::value;
-            if(c < last && part == 5)
-            {
-                const int na = L.win[WIN_LOWER][c], nb = L.win[WIN_TAIL][c];
-                with_window_pair(na, nb, [&](auto NA_, auto NB_) {
-                    constexpr int NA = decltype(NA_)::value, NB = decltype(NB_)::value;
-                    hipLaunchKernelGGL((k_fwd_full_u<NA, NB, VT, XT, RT, R, BS>), grid, dim3(BS), 0, s,
-                                       (int64_t)L.offsets[c], sz, zm, L.ell_col, val, dg, L.desc, r, x, t,
-                                       gate);
-                });
-            }
-            else if(c < last)
-                hipLaunchKernelGGL((k_fwd_full<VT, XT, RT, true, R, BS>), grid, dim3(BS), 0, s,
-                                   (int64_t)L.offsets[c], sz, zm, L.ell_col, val, r, x, t, gate);
-            else
-                hipLaunchKernelGGL((k_fwd_full<VT, XT, RT, false, R, BS>), grid, dim3(BS), 0, s,
-                                   (int64_t)L.offsets[c], sz, zm, L.ell_col, val, r, x, t, gate);
-        });
-    case 3:
-        if(last < 1) return 0;
-        return per_color(L, pr, SH_BWD_FULL, WIN_UPPER, last - 1, 0, -1, [&](auto RR, auto BB, dim3 grid, int c, int64_t sz, ZMap zm) {
-            constexpr int R = decltype(RR)::value, BS = decltype(BB)::value;
-            const int n = L.win[WIN_UPPER][c];
-            with_window(n, [&](auto NN) {
-                constexpr int NS = decltype(NN)::value;
-                hipLaunchKernelGGL((k_bwd_full<NS, VT, XT, R, BS>), grid, dim3(BS), 0, s,
-                                   (int64_t)L.offsets[c], sz, zm, L.ell_col, val, dg, L.desc, (const XT*)t, x, gate);
-            });
-        });
-    }
-    set_error("invalid sweep part");
-    return -2;
 }
 
 int window_slots(int w)
@@ -703,9 +468,8 @@ void window_pair_slots(int wl, int wt, int* a, int* b)
 int launch_sweep(const Level& L, Prec prec, int part, const void* r, bool r_f64, void* x, void* t, hipStream_t s,
                  const int* gate)
 {
-    if(prec == PREC_F64) return sweep_t<double, double, double>(L, part, r, x, t, s, gate);
-    if(r_f64) return sweep_t<__half, float, double>(L, part, r, x, t, s, gate);
-    return sweep_t<__half, float, float>(L, part, r, x, t, s, gate);
+    if(prec == PREC_F64) return sweep_f64(L, part, r, x, t, s, gate);
+    return sweep_mixed(L, part, r, r_f64, x, t, s, gate);
 }
 
 int launch_symgs_zero(const Level& L, Prec prec, const void* r, bool r_f64, void* x, hipStream_t s, const int* gate,
@@ -728,9 +492,16 @@ static int restrict_t(const Level& F, const void* r, const void* x, void* rc, hi
     const int bs = F.shp[std::is_same<VT, double>::value ? PREC_F64 : PREC_MIXED][SH_RESTRICT].block;
     auto go = [&](auto BB) -> int {
         constexpr int BS = decltype(BB)::value;
-        hipLaunchKernelGGL((k_restrict<VT, XT, RT, XT, BS>), dim3(nblk(F.mc, BS)), dim3(BS), 0, s, F.mc,
-                           F.ell_col, vals_of<VT>(F), F.f2c_fine, F.f2c_coarse, (const RT*)r, (const XT*)x,
-                           (XT*)rc, gate);
+        auto run = [&](auto PP) {
+            constexpr bool PAT = decltype(PP)::value;
+            hipLaunchKernelGGL((k_restrict<PAT, VT, XT, RT, XT, BS>), dim3(nblk(F.mc, BS)), dim3(BS), 0, s, F.mc,
+                               F.cols(F.ncolors - 1), vals_of<VT>(F), F.f2c_fine, F.f2c_coarse, (const RT*)r,
+                               (const XT*)x, (XT*)rc, gate);
+        };
+        if(F.use_pat() && F.u_ok)   // every injected row is in the last colour
+            run(std::integral_constant<bool, true>{});
+        else
+            run(std::integral_constant<bool, false>{});
         HPCGX_KCHECK();
         return 0;
     };

@@ -44,6 +44,8 @@ int window_slots(int w);
 void window_pair_slots(int wl, int wt, int* a, int* b);
 // one sweep of a level: 0 zero-guess fwd, 1 zero-guess bwd, 2 fwd keeping t, 3 bwd from t,
 // 4 = 1 also keeping the upper sums outside the last colour in t, 5 = 2 reusing them
+int sweep_f64(const Level& L, int part, const void* r, void* x, void* t, hipStream_t s, const int* gate);
+int sweep_mixed(const Level& L, int part, const void* r, bool r_f64, void* x, void* t, hipStream_t s, const int* gate);
 int launch_sweep(const Level& L, Prec prec, int part, const void* r, bool r_f64, void* x, void* t, hipStream_t s,
                  const int* gate);
 // u (may be null): also keep the upper sums outside the last colour, for a

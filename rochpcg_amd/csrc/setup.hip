@@ -496,6 +496,13 @@ int color_level(Level& L, hipStream_t s)
     return 0;
 }
 
+struct ColorRanges
+{
+    int off[MAX_COLORS + 1];
+};
+constexpr uint8_t PAT_NONE = 255;   // no pattern yet
+static_assert(PAT_MAX < PAT_NONE, "pattern ids are one byte");
+
 // Window statistics of one colour's rows [off, off+size): the largest lower
 // count d, upper count W - us and last-colour count W - tl (stats[0..2]).
 __global__ __launch_bounds__(256) void k_window_stats(int64_t off, int64_t size, const int32_t* __restrict__ desc,
@@ -548,6 +555,102 @@ static int window_stats(Level& L, hipStream_t s)
     return 0;
 }
 
+// One round of the pattern search: for every colour (grid.y) the first row
+// without a pattern, rep[c], stands for pattern `k`; its rows without one that
+// have the same offsets and descriptor get it, and next[c] becomes the first
+// row still without one (INT_MAX: none).
+__global__ __launch_bounds__(256) void k_pattern_round(ColorRanges cr, int k, const int32_t* __restrict__ col,
+                                                       const int32_t* __restrict__ desc,
+                                                       const int32_t* __restrict__ rep, int32_t* __restrict__ next,
+                                                       uint8_t* __restrict__ pat, int32_t* __restrict__ tab)
+{
+    const int c = blockIdx.y;
+    const int32_t q = rep[c];
+    if(q == INT_MAX) return;
+    const int64_t off = cr.off[c], end = cr.off[c + 1];
+    if(blockIdx.x == 0 && threadIdx.x <= W)
+    {
+        const int p = threadIdx.x;
+        int32_t* t = tab + ((int64_t)c * PAT_MAX + k) * (PAT_QUADS * 4);
+        if(p == W)
+            t[p] = desc[q];
+        else
+        {
+            const int32_t v = col[ell_at(p, q)];
+            t[p] = v < 0 ? 0 : v - q;
+        }
+    }
+    int first = INT_MAX;
+    const int32_t qd = desc[q];
+    for(int64_t r = off + (int64_t)blockIdx.x * 256 + threadIdx.x; r < end; r += (int64_t)gridDim.x * 256)
+    {
+        if(k > 0 && pat[r] != PAT_NONE) continue;
+        bool same = desc[r] == qd;
+        for(int p = 0; p < W && same; ++p)
+        {
+            const int32_t a = col[ell_at(p, r)], b = col[ell_at(p, q)];
+            same = (a < 0) == (b < 0) && (a < 0 || a - (int32_t)r == b - q);
+        }
+        pat[r] = same ? (uint8_t)k : PAT_NONE;
+        if(!same && (int)r < first) first = (int)r;
+    }
+    for(int o = 32; o > 0; o >>= 1) first = min(first, __shfl_xor(first, o, 64));
+    if((threadIdx.x & 63) == 0 && first != INT_MAX) atomicMin(next + c, first);
+}
+
+// Row patterns of a level (Level::pat, Cols<true>) from its columns and
+// descriptors: at most PAT_MAX rounds over the rows, the first of which reads
+// every column once (0.8 ms at 320^3) and the others only rows still without a
+// pattern.  A level with a colour of more than PAT_MAX patterns (odd grids,
+// where the colours' sub-grids differ in size) keeps the column array alone; so
+// does one of 2^29 rows or more, whose f64 gather offsets exceed 32 bits.
+static int build_patterns(Level& L, hipStream_t s)
+{
+    const int nc = L.ncolors;
+    if(L.m >= ((int64_t)1 << 29)) return 0;
+    DevTemp tpat, ttab, trep;
+    const size_t tab_bytes = sizeof(int32_t) * PAT_QUADS * 4 * PAT_MAX * nc;
+    HPCGX_HIP(hipMalloc(&tpat.p, (size_t)L.m));
+    HPCGX_HIP(hipMalloc(&ttab.p, tab_bytes));
+    HPCGX_HIP(hipMemsetAsync(ttab.p, 0, tab_bytes, s));
+    // the representatives of every round; round k + 1's are round k's `next`
+    std::vector<int32_t> rep((size_t)nc * (PAT_MAX + 1), INT_MAX);
+    ColorRanges cr;
+    int mx = 0;
+    for(int c = 0; c <= nc; ++c) cr.off[c] = L.offsets[c];
+    for(int c = 0; c < nc; ++c)
+    {
+        rep[c] = L.sizes[c] > 0 ? L.offsets[c] : INT_MAX;
+        mx = std::max(mx, L.sizes[c]);
+    }
+    HPCGX_HIP(hipMalloc(&trep.p, sizeof(int32_t) * rep.size()));
+    int32_t* d = (int32_t*)trep.p;
+    HPCGX_HIP(hipMemcpyAsync(d, rep.data(), sizeof(int32_t) * rep.size(), hipMemcpyHostToDevice, s));
+    const dim3 grid((unsigned)std::min<int64_t>(1024, ceil_div(mx, 256)), (unsigned)nc);
+    for(int k = 0; k < PAT_MAX; ++k)
+    {
+        hipLaunchKernelGGL(k_pattern_round, grid, dim3(256), 0, s, cr, k, L.ell_col, L.desc,
+                           (const int32_t*)d + (size_t)k * nc, d + (size_t)(k + 1) * nc, (uint8_t*)tpat.p,
+                           (int32_t*)ttab.p);
+        HPCGX_HIP(hipGetLastError());
+        // eight rounds settle a parity colouring; look again after each later one
+        if(k < 7) continue;
+        HPCGX_HIP(hipMemcpyAsync(rep.data(), d, sizeof(int32_t) * rep.size(), hipMemcpyDeviceToHost, s));
+        HPCGX_HIP(hipStreamSynchronize(s));
+        bool left = false;
+        for(int c = 0; c < nc; ++c) left = left || rep[(size_t)(k + 1) * nc + c] != INT_MAX;
+        if(left) continue;
+        L.npat = 0;
+        for(int j = 0; j <= k; ++j)
+            for(int c = 0; c < nc; ++c)
+                if(rep[(size_t)j * nc + c] != INT_MAX) L.npat = j + 1;
+        L.pat = (uint8_t*)tpat.release();
+        L.pat_tab = (int32_t*)ttab.release();
+        return 0;
+    }
+    return 0;
+}
+
 int build_level(Level& L, int nx, int ny, int nz, bool with_f64, bool with_f16, hipStream_t s)
 {
     L.nx = nx;
@@ -589,7 +692,8 @@ int build_level(Level& L, int nx, int ny, int nz, bool with_f64, bool with_f16, 
     HPCGX_HIP(hipStreamSynchronize(s));
     HPCGX_HIP(hipFree(L.iperm_tmp));
     L.iperm_tmp = nullptr;
-    return window_stats(L, s);
+    HPCGX_TRY(window_stats(L, s));
+    return build_patterns(L, s);
 }
 
 int build_transfer(Level& F, Level& C, hipStream_t s)
@@ -632,6 +736,8 @@ void free_level(Level& L)
     f(L.ell_h);
     f(L.diag_idx);
     f(L.desc);
+    f(L.pat);
+    f(L.pat_tab);
     f(L.inv_diag);
     f(L.diag64);
     f(L.diag_h);

@@ -105,7 +105,8 @@ int problem_create(Problem*& out, int nx, int ny, int nz, int nlevels, bool with
     if(with_mixed && alloc((void**)&P->z32, m0 * 4)) return fail(-1);
     P->hist_cap = 4096;
     // a batched fused SpMV + dot keeps one partial per 64-row block
-    P->partial_cap = std::max<int64_t>(FOLD_MAX, (int64_t)(m0 / 64) + 64);
+    // (each colour rounded up to whole blocks)
+    P->partial_cap = std::max<int64_t>(FOLD_MAX, (int64_t)(m0 / 64) + MAX_COLORS);
     if(alloc((void**)&P->sc, sizeof(CGScalars)) || alloc((void**)&P->hist, sizeof(double) * (P->hist_cap + 1)) ||
        alloc((void**)&P->partial, sizeof(double) * P->partial_cap) ||
        alloc((void**)&P->dout, 8 * sizeof(double)))
@@ -488,15 +489,19 @@ int cg_solve(Problem& P, int mode, bool precond, const double* b, double* x, int
 }
 
 // Algorithmic HBM bytes of one V-cycle from level l down, as this library's
-// kernels run it: every slot a kernel loads once (4 B column + value; a sweep
-// loads its colour's window bucket for each row), neighbour x
-// gathers served from cache, own-row vectors read and written once.
-static double vcycle_bytes(const Problem& P, int l, bool mixed)
+// kernels run it: every slot a kernel loads once (a sweep loads its colour's
+// window bucket for each row), neighbour x gathers served from cache, own-row
+// vectors read and written once.  A slot counts 4 B of column and its value and
+// a sweep's row 4 B of descriptor, the ELL's own bytes; with `stream` set, what
+// the kernels load where the level has row patterns: the value alone, and one
+// byte a row for columns and descriptor.
+static double vcycle_bytes(const Problem& P, int l, bool mixed, bool stream)
 {
     const Level& L = P.L[l];
-    const double ib = 4.0, vb = mixed ? 2.0 : 8.0, xb = mixed ? 4.0 : 8.0;
+    const bool pat = stream && L.use_pat();
+    const double vb = mixed ? 2.0 : 8.0, xb = mixed ? 4.0 : 8.0;
     const double rb = (l == 0) ? 8.0 : xb;   // the CG residual is f64
-    const double slot = ib + vb;
+    const double slot = vb + (pat ? 0.0 : 4.0), head = pat ? 1.0 : 4.0, full = stream ? head : 0.0;
     const int last = L.ncolors - 1;
     const bool coarsest = l + 1 >= P.nlevels;
     const bool keep_u = !coarsest && L.u_ok;
@@ -504,13 +509,13 @@ static double vcycle_bytes(const Problem& P, int l, bool mixed)
     for(int c = 0; c <= last; ++c)
     {
         const double n = L.sizes[c];
-        b += window_slots(L.win[WIN_LOWER][c]) * n * slot + n * (4 + vb + rb + xb);   // fwd_zero
-        if(c < last) b += window_slots(L.win[WIN_UPPER][c]) * n * slot + n * (4 + vb + 2 * xb + (keep_u ? xb : 0));   // bwd_zero
+        b += window_slots(L.win[WIN_LOWER][c]) * n * slot + n * (head + vb + rb + xb);   // fwd_zero
+        if(c < last) b += window_slots(L.win[WIN_UPPER][c]) * n * slot + n * (head + vb + 2 * xb + (keep_u ? xb : 0));   // bwd_zero
     }
     if(coarsest) return b;
     const double mc = (double)L.mc;
-    b += mc * (W * slot + rb + 4 + 4 + xb);   // fused residual + restriction (whole rows)
-    b += vcycle_bytes(P, l + 1, mixed);
+    b += mc * (W * slot + full + rb + 4 + 4 + xb);   // fused residual + restriction (whole rows)
+    b += vcycle_bytes(P, l + 1, mixed, stream);
     b += mc * (4 + 4 + 3 * xb);                // prolongation
     for(int c = 0; c <= last; ++c)
     {
@@ -519,28 +524,29 @@ static double vcycle_bytes(const Problem& P, int l, bool mixed)
         {
             int na = 0, nb = 0;
             window_pair_slots(L.win[WIN_LOWER][c], L.win[WIN_TAIL][c], &na, &nb);
-            b += (na + nb) * n * slot + n * (4 + vb + rb + 3 * xb);
+            b += (na + nb) * n * slot + n * (head + vb + rb + 3 * xb);
         }
         else
-            b += n * (W * slot + rb + xb + (c < last ? xb : 0));   // whole-row forward sweep
-        if(c < last) b += window_slots(L.win[WIN_UPPER][c]) * n * slot + n * (4 + vb + 2 * xb);   // bwd_full
+            b += n * (W * slot + full + rb + xb + (c < last ? xb : 0));   // whole-row forward sweep
+        if(c < last) b += window_slots(L.win[WIN_UPPER][c]) * n * slot + n * (head + vb + 2 * xb);   // bwd_full
     }
     return b;
 }
 
-int iteration_bytes(const Problem& P, int mode, double* vcycle, double* iteration)
+int iteration_bytes(const Problem& P, int mode, bool stream, double* vcycle, double* iteration)
 {
-    const bool mixed = mode == CG_MIXED;
-    const double mg = vcycle_bytes(P, 0, mixed);
+    const bool mixed = mode == CG_MIXED, pat = stream && P.L[0].use_pat();
+    const double mg = vcycle_bytes(P, 0, mixed, stream);
     const double m0 = (double)P.L[0].m;
     const double vb = mixed ? 2.0 : 8.0, zb = mixed ? 4.0 : 8.0;
+    const double spmv = m0 * (W * (vb + (pat ? 0.0 : 4.0)) + (stream ? (pat ? 1.0 : 4.0) : 0.0) + 16);
     double it = mg;
-    it += m0 * (W * (4 + vb) + 16);            // SpMV + p'Ap
+    it += spmv;                                // SpMV + p'Ap
     it += m0 * (8 + zb);                       // r'z
     it += m0 * (zb + 32);                      // x += alpha p (deferred), p = z + beta p
     it += m0 * 24;                             // r update and ||r||
     if(mixed && P.replace_every > 0)           // true residual every k iterations
-        it += m0 * (W * (4 + vb) + 16 + 24 + 16) / P.replace_every;
+        it += (spmv + m0 * (24 + 16)) / P.replace_every;
     if(vcycle) *vcycle = mg;
     if(iteration) *iteration = it;
     return 0;
@@ -554,6 +560,7 @@ int64_t problem_device_bytes(const Problem& P)
         const Level& L = P.L[l];
         const int64_t m = L.m, me = ell_rows(m);
         b += 4 * W * me + 4 * 4 * m;   // columns; diag_idx, desc, perm, colors
+        if(L.pat) b += m + (int64_t)4 * PAT_QUADS * 4 * PAT_MAX * L.ncolors;   // row patterns
         if(P.has_f64) b += 8 * W * me + 8 * m + 8 * m + (l > 0 ? 16 * m : 0);   // values, 1/a_ii, t, r, x
         if(P.has_mixed) b += 2 * W * me + 4 * m + 4 * m + (l > 0 ? 8 * m : 0);
         b += 3 * 4 * L.mc;   // transfer maps
