@@ -259,7 +259,8 @@ int hpcgx_batch_cg(hpcgx_batch* b, int mode, int max_iter, double tolerance, int
  * milliseconds of the launches of kind k over the iterations -- 0 SpMV,
  * 1/2 zero-guess forward/backward sweeps, 3/4 forward/backward sweeps,
  * 5 restriction, 6 prolongation, 7 dot, 8 p update, 9 x/r update, 10 copy,
- * 11 waxpby -- kind_bytes[k] = their algorithmic HBM bytes per iteration,
+ * 11 waxpby; the launch of the problems' coarse levels
+ * (hpcgx_set_coarse_rows) counts as kind 1 -- kind_bytes[k] = their algorithmic HBM bytes per iteration,
  * *iter_ms = milliseconds per iteration (no reference counterpart) */
 int hpcgx_batch_profile(hpcgx_batch* b, int mode, int iters, double* kind_ms, double* kind_bytes, double* iter_ms);
 /* residual history of problem k's last batched CG: normr after iterations
@@ -306,6 +307,14 @@ int hpcgx_set_sweep_columns(hpcgx_problem* p, int level, int columns);
  * its colours repeats at most 32 lists, as the parity colourings of even grids
  * do; other levels always read the column array.  level -1 applies to all. */
 int hpcgx_set_row_patterns(hpcgx_problem* p, int level, int on);
+/* The V-cycle runs the levels of at most `rows` rows, together with all below
+ * them, as one launch of one workgroup (no reference counterpart; a tuning
+ * knob).  -1 = the default (5000 rows for the f64 store, 8191 for the mixed
+ * one), 0 = every level as launches per colour.  A level whose x and row sums
+ * do not fit a CU's LDS, or of a colouring with too many entries on both sides
+ * of the diagonal, is run as launches whatever `rows` says.  Results do not
+ * depend on it. */
+int hpcgx_set_coarse_rows(hpcgx_problem* p, int rows);
 int hpcgx_synchronize(hpcgx_problem* p);
 int hpcgx_malloc(void** ptr, size_t bytes);
 int hpcgx_free(void* ptr);

@@ -90,6 +90,7 @@ def _load():
         "hpcgx_set_shape": ([vp, i32, i32, i32, i32, i32], i32),
         "hpcgx_set_sweep_columns": ([vp, i32, i32], i32),
         "hpcgx_set_row_patterns": ([vp, i32, i32], i32),
+        "hpcgx_set_coarse_rows": ([vp, i32], i32),
         "hpcgx_get_shape": ([vp, i32, i32, i32, P(i32), P(i32)], i32),
         "hpcgx_synchronize": ([vp], i32),
         "hpcgx_batch_create": ([i32, vp, i32, i32, vp, P(vp)], i32),
@@ -420,6 +421,11 @@ class Problem:
         """Read columns from the row patterns (True) or from the column array
         (False) where a level has both (results do not change)."""
         _check(lib.hpcgx_set_row_patterns(self.h, level, int(bool(on))))
+
+    def set_coarse_rows(self, rows=-1):
+        """Largest level the V-cycle runs, with all below it, in one workgroup
+        (-1: the default, 0: none; results do not change)."""
+        _check(lib.hpcgx_set_coarse_rows(self.h, rows))
 
     def get_shape(self, level, op, mixed=False):
         b, r = C.c_int(), C.c_int()

@@ -4,6 +4,7 @@
 // across all problems.  Blocks find their (problem, row block) segment in a
 // device table; reductions, CG scalars and convergence flags stay per problem.
 #pragma once
+#include "coarse.hpp"
 #include "solver.hpp"
 
 namespace hpcgx
@@ -104,6 +105,8 @@ enum BKind : int
     BK_CG_XR,         // x += alpha p, r -= alpha Ap, ||r||
     BK_COPY,          // w = a
     BK_WAXPBY,        // w = alpha a + beta b (alpha == 1 form only: b - A x)
+    BK_COUNT,
+    BK_COARSE = BK_COUNT   // the problems' coarse levels, one workgroup each (coarse.hip)
 };
 
 struct BLaunch
@@ -125,9 +128,12 @@ struct BLaunch
     double alpha, beta;
     int64_t nrows;    // rows (elements) over all segments
     int any_t;        // some segment keeps or reads SymGS partial sums (BSeg::t)
+    CoarseRun* runs;  // BK_COARSE: device table of nseg runs, the LDS they take,
+    size_t lds;       // and their algorithmic bytes
+    double bytes;
 };
 
-constexpr int BK_COUNT = 12;
+static_assert(BK_COUNT == 12, "hpcgx_batch_profile reports 12 kinds");
 
 struct Batch
 {
@@ -137,7 +143,7 @@ struct Batch
     bool own_stream = false;
     int block[MAX_LEVELS] = {256, 256, 256, 256, 256, 256, 256, 256};
     int rows[MAX_LEVELS] = {1, 1, 1, 1, 1, 1, 1, 1};   // sweeps: rows per thread, per level
-    std::vector<BSeg*> tables;              // device allocations of the plans
+    std::vector<void*> tables;              // device allocations of the plans
     std::vector<BLaunch> pre[2], iter[2];   // preamble and one iteration, per CG mode
     bool planned = false;
     hipGraph_t graph[2] = {nullptr, nullptr};

@@ -7,6 +7,7 @@
 #include <string>
 
 #include "batch.hpp"
+#include "coarse.hpp"
 #include "ops.hpp"
 #include "refpath.hpp"
 #include "setup.hpp"
@@ -610,6 +611,19 @@ int hpcgx_set_row_patterns(hpcgx_problem* p, int level, int on)
     }
     for(int l = 0; l < p->P->nlevels; ++l)
         if(level < 0 || l == level) p->P->L[l].pat_off = on == 0;
+    p->P->invalidate_graphs();
+    return 0;
+}
+
+int hpcgx_set_coarse_rows(hpcgx_problem* p, int rows)
+{
+    CHECK_P(p);
+    if(rows < -1)
+    {
+        set_error("invalid row count");
+        return -2;
+    }
+    p->P->coarse_rows = rows;
     p->P->invalidate_graphs();
     return 0;
 }

@@ -1,0 +1,67 @@
+// coarse.hpp -- the bottom of the V-cycle as one launch (coarse.hip).
+#pragma once
+#include "solver.hpp"
+
+namespace hpcgx
+{
+
+// Sections of a row's entries: left of the diagonal, right of it, and of these
+// the ones outside and inside the last colour.
+enum CoarseSection : int
+{
+    SEC_LOWER = 0,
+    SEC_UPPER = 1,
+    SEC_MID = 2,
+    SEC_TAIL = 3,
+    SEC_COUNT = 4
+};
+
+// One step of a symmetric Gauss-Seidel sweep over a level: some rows of one
+// colour, and the slot groups (of four) its one or two sums take.
+struct CoarseStep
+{
+    int kind;       // CoarseKind
+    int off, n;     // rows [off, off + n), at most a team's threads
+    int va, ia, na; // first sum: its first group among the values and among the
+                    // columns (section * groups + group), and how many
+    int vb, ib, nb; // second sum
+};
+
+// What one workgroup needs of a level, in device memory (coarse_build).
+struct CoarseLevel
+{
+    const void* val;           // values, and diagonal
+    const void* dg;
+    const uint2* at;           // LDS byte offsets of the columns' x, 16 bits each: [section][group][row]
+    const int32_t* f2c_fine;   // to the next level
+    const int32_t* f2c_coarse;
+    const CoarseStep* steps;   // pre-smoothing steps, then post-smoothing ones
+    void* r;                   // the level's vectors (level 0: given with the launch)
+    void* x;
+    int m, mc, npre, npost;
+    int lds_x, lds_t;          // where the level's x and t lie in LDS (bytes)
+};
+
+// One V-cycle from lv[0] down over nl levels: x = M^-1 r.
+struct CoarseRun
+{
+    const CoarseLevel* lv;
+    int nl;
+    int r_f64;                 // r is f64 whatever the vector type
+    const void* r;
+    void* x;
+    const int* gate;
+};
+
+// build the plans of a problem whose levels and vectors exist
+int coarse_build(Problem& P);
+void coarse_free(Problem& P);
+// the first level that runs in one workgroup, with everything below it
+// (nlevels: none)
+int coarse_first(const Problem& P, Prec prec);
+CoarseRun coarse_run(const Problem& P, int l, Prec prec, const void* r, bool r_f64, void* x, const int* gate);
+int launch_coarse(const CoarseRun& run, Prec prec, size_t lds, hipStream_t s);
+// the same for `n` problems, one workgroup each (runs in device memory)
+int launch_coarse_batch(const CoarseRun* runs, int n, Prec prec, size_t lds, hipStream_t s);
+
+}  // namespace hpcgx

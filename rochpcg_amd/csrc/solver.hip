@@ -12,6 +12,7 @@
 // per iteration.  A `done` flag written by the ||r|| reduction gates every
 // kernel of later iterations, so iterations can be enqueued (or replayed as a
 // captured hipGraph) ahead of the convergence test.
+#include "coarse.hpp"
 #include "refpath.hpp"
 #include "setup.hpp"
 #include "solver.hpp"
@@ -113,6 +114,7 @@ int problem_create(Problem*& out, int nx, int ny, int nz, int nlevels, bool with
         return fail(-1);
     if(hipMemsetAsync(P->sc, 0, sizeof(CGScalars), P->s) != hipSuccess)
         return fail(-1);
+    if(coarse_build(*P)) return fail(-1);
     if(make_rhs(P->L[0], 0, 0, P->b, P->xexact, P->x, P->s)) return fail(-1);
     if(hipStreamSynchronize(P->s) != hipSuccess)
     {
@@ -128,6 +130,7 @@ void problem_destroy(Problem* P)
     if(!P) return;
     if(P->s) (void)hipStreamSynchronize(P->s);
     refpath_free(*P);
+    coarse_free(*P);
     for(int g = 0; g < 2; ++g)
     {
         if(P->gexec[g]) (void)hipGraphExecDestroy(P->gexec[g]);
@@ -195,6 +198,8 @@ int mg(Problem& P, int l, Prec prec, const void* r, bool r_f64, void* x, const i
 {
     Level& F = P.L[l];
     LevelVecs* V = (prec == PREC_F64) ? P.v64 : P.v32;
+    if(l >= coarse_first(P, prec))
+        return launch_coarse(coarse_run(P, l, prec, r, r_f64, x, gate), prec, P.coarse[prec].lds[l], P.s);
     if(l + 1 < P.nlevels)
     {
         LevelVecs& C = V[l + 1];
@@ -495,7 +500,7 @@ int cg_solve(Problem& P, int mode, bool precond, const double* b, double* x, int
 // a sweep's row 4 B of descriptor, the ELL's own bytes; with `stream` set, what
 // the kernels load where the level has row patterns: the value alone, and one
 // byte a row for columns and descriptor.
-static double vcycle_bytes(const Problem& P, int l, bool mixed, bool stream)
+double vcycle_bytes(const Problem& P, int l, bool mixed, bool stream)
 {
     const Level& L = P.L[l];
     const bool pat = stream && L.use_pat();

@@ -31,6 +31,22 @@ struct LevelVecs
 };
 
 struct RefPath;
+struct CoarseLevel;
+
+// a problem's coarse levels in one precision, as one workgroup runs them (coarse.hip)
+struct CoarsePlan
+{
+    int first = MAX_LEVELS;        // first level that can run so
+    void* mem = nullptr;           // descriptions, steps and columns
+    CoarseLevel* lv = nullptr;     // of level `first`
+    size_t lds[MAX_LEVELS] = {};   // LDS of a run from each level
+};
+// Levels of at most this many rows run so, [precision].  One workgroup streams a
+// level's values at one CU's rate, launches at the GPU's: at 4096 rows it takes
+// 16 us less for the coarsest level of an FP64 V-cycle and 21 us less for that
+// of a mixed one, at 5832 rows 9 us more and 16 us less, at 8000 rows 66 us more
+// and 5 us less (the f16 values are a quarter of the bytes).
+constexpr int COARSE_ROWS[2] = {5000, 8191};
 
 struct Problem
 {
@@ -70,6 +86,8 @@ struct Problem
     int graph_mode = -1;
     bool graph_precond = true;
     int graph_replace = -1;
+    CoarsePlan coarse[2];     // [precision]
+    int coarse_rows = -1;     // levels of at most this many rows run in one workgroup (-1: COARSE_ROWS)
     RefPath* ref = nullptr;   // natural-order work vectors of the reference path (refpath.hip)
 
     // forget captured graphs (launch shapes or operands changed)
@@ -103,6 +121,7 @@ int cg_end(Problem& P, int* niters, double* normr, double* normr0, double* histo
 int64_t problem_device_bytes(const Problem& P);
 // algorithmic HBM bytes of one V-cycle and of one CG iteration in `mode`: the
 // ELL's bytes of the slots the kernels use, or (stream) what they load
+double vcycle_bytes(const Problem& P, int l, bool mixed, bool stream);
 int iteration_bytes(const Problem& P, int mode, bool stream, double* vcycle, double* iteration);
 int cg_solve(Problem& P, int mode, bool precond, const double* b, double* x, int max_iter, double tol,
              bool use_graph, int* niters, double* normr, double* normr0, double* history, int hist_len);
