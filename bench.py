@@ -239,7 +239,7 @@ def main():
     ap.add_argument("--cpu-iters", type=int, default=5)
     ap.add_argument("--cpu-nx", type=int, default=320, help="cube side of the bounded CPU-baseline sample")
     ap.add_argument("--eager", action="store_true", help="launch kernels one by one instead of a hipGraph")
-    ap.add_argument("--no-tune", action="store_true", help="keep the default launch shapes (256 threads, 1 row)")
+    ap.add_argument("--no-tune", action="store_true", help="keep the default launch shapes")
     ap.add_argument("--no-batch", action="store_true", help="skip the batched uneven-problems leg")
     ap.add_argument("--batch-count", type=int, default=64)
     ap.add_argument("--shapes", default=None,

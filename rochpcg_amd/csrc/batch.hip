@@ -316,6 +316,13 @@ struct Planner
         return l;
     }
 
+    int block(int l)
+    {
+        int64_t m = 0;
+        for(const Problem* P : B.probs) m += P->L[l].m;
+        return B.block[l] ? B.block[l] : default_block(m);
+    }
+
     int max_colors(int l)
     {
         int n = 0;
@@ -350,7 +357,7 @@ struct Planner
     // the V-cycle from level l (ComputeMG.cpp:64-102), all problems in lockstep
     int mg(int l)
     {
-        const int bs = B.block[l];
+        const int bs = block(l);
         const bool last = (l + 1 == B.nlevels);
         const int r64 = (l == 0) ? 1 : (prec == PREC_F64);
         if(l >= coarse_from()) return coarse(l);
@@ -448,7 +455,7 @@ struct Planner
     int outer_spmv(bool dot, bool from_x, bool into_tmp)
     {
         next_subs = max_colors(0);   // one segment per colour: a block stages one colour's patterns
-        return add(BK_SPMV, B.block[0], false, 1, dot ? 1 : 0, 0.0, [&](int k, BSeg& s) {
+        return add(BK_SPMV, block(0), false, 1, dot ? 1 : 0, 0.0, [&](int k, BSeg& s) {
             Problem* P = B.probs[k];
             const Level& L = P->L[0];
             if(sub >= L.ncolors) return false;

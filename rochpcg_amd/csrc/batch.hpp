@@ -141,7 +141,7 @@ struct Batch
     int nlevels = 0;
     hipStream_t s = nullptr;
     bool own_stream = false;
-    int block[MAX_LEVELS] = {256, 256, 256, 256, 256, 256, 256, 256};
+    int block[MAX_LEVELS] = {};                        // threads per block (0: default_block of the launch's rows)
     int rows[MAX_LEVELS] = {1, 1, 1, 1, 1, 1, 1, 1};   // sweeps: rows per thread, per level
     std::vector<void*> tables;              // device allocations of the plans
     std::vector<BLaunch> pre[2], iter[2];   // preamble and one iteration, per CG mode

@@ -57,6 +57,16 @@ struct Shape
     int rows = 1;      // consecutive rows per thread: 1 or 2
 };
 
+// Default threads per block of the launches over levels of m rows in all.
+// A colour of a small level is a few hundred waves: in blocks of one wave they
+// spread over all CUs, and a wave waits for its own row patterns only (104^3
+// FP64: 64 threads 568 us an iteration, 128 581, 256 638; 32^3 218, 227, 240).
+// From about 2^21 rows on every CU has blocks enough either way, and larger ones
+// stage the patterns less often (320^3 mixed: 3046, 2985, 2943; at 128^3 and
+// 160^3 the two are within 1-4%).
+constexpr int64_t SMALL_ROWS = (int64_t)1 << 21;
+inline int default_block(int64_t m) { return m <= SMALL_ROWS ? 64 : 256; }
+
 // Block-to-tile order of one colour launch of a sweep.  k <= 1: tile = block.
 // k > 1: the colour's tiles form `planes` planes of k columns of tpc tiles
 // each (in row order); block b takes column b / (planes*tpc), plane

@@ -651,12 +651,31 @@ static int build_patterns(Level& L, hipStream_t s)
     return 0;
 }
 
+// Launch shapes until the autotuner sets others.  Two rows a thread halve the
+// load instructions of a row; on large levels that is worth it where the
+// registers still let enough waves in flight: the SpMV (320^3: FP64 1.667 ->
+// 1.582 ms, mixed 0.755 -> 0.728 ms) and the FP64 forward sweeps (0.903 -> 0.863
+// and 1.209 -> 1.181 ms), not the backward ones (0.896 -> 0.940 ms) nor the mixed
+// ones (0.297 -> 0.366 ms).
+static void default_shapes(Level& L)
+{
+    const int block = default_block(L.m);
+    for(int p = 0; p < 2; ++p)
+        for(int o = 0; o < SH_COUNT; ++o)
+        {
+            const bool fwd = o == SH_FWD_ZERO || o == SH_FWD_ZERO_N || o == SH_FWD_FULL || o == SH_FWD_FULL_N;
+            L.shp[p][o].block = block;
+            L.shp[p][o].rows = L.m > SMALL_ROWS && (o == SH_SPMV || (p == PREC_F64 && fwd)) ? 2 : 1;
+        }
+}
+
 int build_level(Level& L, int nx, int ny, int nz, bool with_f64, bool with_f16, hipStream_t s)
 {
     L.nx = nx;
     L.ny = ny;
     L.nz = nz;
     L.m = (int64_t)nx * ny * nz;
+    default_shapes(L);
     if(L.m <= 0 || L.m > INT_MAX)
     {
         set_error("level size out of range");
