@@ -302,8 +302,9 @@ static RedArgs store_red(Problem* P)
     RedArgs ra;
     ra.partial = P->partial;
     ra.op = OP_STORE;
-    ra.out = P->dout;
+    ra.out = P->h_out;
     ra.cap = P->partial_cap;
+    ra.ticket = P->ticket;
     return ra;
 }
 
@@ -314,7 +315,6 @@ int hpcgx_dot(hpcgx_problem* p, int64_t n, const double* x, const double* y, dou
     if(n > 0) CHECK_PTRS(x, y);
     Problem* P = p->P;
     HPCGX_TRY(launch_dot(n, x, true, y, true, store_red(P), P->s, nullptr));
-    HPCGX_HIP(hipMemcpyAsync(P->h_out, P->dout, sizeof(double), hipMemcpyDeviceToHost, P->s));
     HPCGX_HIP(hipStreamSynchronize(P->s));
     *result = P->h_out[0];
     return 0;
@@ -333,8 +333,7 @@ int hpcgx_residual(hpcgx_problem* p, int64_t n, const double* v1, const double* 
     CHECK_PTRS(result);
     if(n > 0) CHECK_PTRS(v1, v2);
     Problem* P = p->P;
-    HPCGX_TRY(launch_absdiff_max(n, v1, v2, P->partial, P->partial_cap, P->dout, P->s));
-    HPCGX_HIP(hipMemcpyAsync(P->h_out, P->dout, sizeof(double), hipMemcpyDeviceToHost, P->s));
+    HPCGX_TRY(launch_absdiff_max(n, v1, v2, P->partial, P->partial_cap, P->h_out, P->s));
     HPCGX_HIP(hipStreamSynchronize(P->s));
     *result = P->h_out[0];
     return 0;
@@ -354,7 +353,6 @@ int hpcgx_fused_waxpby_dot(hpcgx_problem* p, int64_t n, double alpha, const doub
     if(n > 0) CHECK_PTRS(x, y);
     Problem* P = p->P;
     HPCGX_TRY(launch_axpy_dot(n, alpha, x, y, store_red(P), P->s, nullptr));
-    HPCGX_HIP(hipMemcpyAsync(P->h_out, P->dout, sizeof(double), hipMemcpyDeviceToHost, P->s));
     HPCGX_HIP(hipStreamSynchronize(P->s));
     *result = P->h_out[0];
     return 0;

@@ -34,8 +34,8 @@ struct Context
 {
     hipStream_t s = nullptr;
     double* partial = nullptr;
-    double* dout = nullptr;
-    double h_out = 0.0;
+    int* ticket = nullptr;
+    double* h_out = nullptr;   // pinned: the kernels write results there
     int device = -1;
     bool ok = false;
 };
@@ -53,11 +53,12 @@ Context& ctx()
     {
         if(hipGetDevice(&c.device) != hipSuccess || hipStreamCreateWithFlags(&c.s, hipStreamNonBlocking) != hipSuccess ||
            hipMalloc(&c.partial, sizeof(double) * FOLD_MAX) != hipSuccess ||
-           hipMalloc(&c.dout, 8 * sizeof(double)) != hipSuccess)
+           hipMalloc(&c.ticket, sizeof(int)) != hipSuccess || hipMemset(c.ticket, 0, sizeof(int)) != hipSuccess ||
+           hipHostMalloc((void**)&c.h_out, sizeof(double), hipHostMallocDefault) != hipSuccess)
         {
             fprintf(stderr, "rochpcg_amd: cannot initialise the HIP context\n");
             // release what was made, so that a later call starts clean
-            if(c.dout) (void)hipFree(c.dout);
+            if(c.ticket) (void)hipFree(c.ticket);
             if(c.partial) (void)hipFree(c.partial);
             if(c.s) (void)hipStreamDestroy(c.s);
             c = Context();
@@ -92,17 +93,17 @@ RedArgs store_red()
     RedArgs ra;
     ra.partial = ctx().partial;
     ra.op = OP_STORE;
-    ra.out = ctx().dout;
+    ra.out = ctx().h_out;
     ra.cap = FOLD_MAX;
+    ra.ticket = ctx().ticket;
     return ra;
 }
 
 int fetch_result(double& result)
 {
     Context& c = ctx();
-    HPCGX_HIP(hipMemcpyAsync(&c.h_out, c.dout, sizeof(double), hipMemcpyDeviceToHost, c.s));
     HPCGX_HIP(hipStreamSynchronize(c.s));
-    result = c.h_out;
+    result = *c.h_out;
     return 0;
 }
 
@@ -557,7 +558,7 @@ int ComputeResidual(const local_int_t n, const Vector& v1, const Vector& v2, dou
         return 1;
     Context& c = ctx();
     if(!c.ok) return 1;
-    if(launch_absdiff_max(n, v1.d_values, v2.d_values, c.partial, FOLD_MAX, c.dout, c.s)) return 1;
+    if(launch_absdiff_max(n, v1.d_values, v2.d_values, c.partial, FOLD_MAX, c.h_out, c.s)) return 1;
     return fetch_result(residual) ? 1 : 0;
 }
 

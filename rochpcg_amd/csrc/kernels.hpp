@@ -108,6 +108,45 @@ __device__ __forceinline__ void fold_partials(const double* __restrict__ partial
     if(threadIdx.x == 0) apply_op(ra.op, s, ra.sc, ra.hist, ra.hist_cap, ra.out);
 }
 
+// Both phases in one launch: the block that takes the last ticket folds all the
+// partials, in the grouping of fold_partials (one partial a thread).  Device-scope
+// stores and loads of the partials, ordered by the ticket, carry them across the
+// XCDs' L2s; no block waits for another.
+template <int BS>
+__device__ __forceinline__ void block_total(double v, const RedArgs& ra)
+{
+    __shared__ double lds[BS / 64];
+    __shared__ int last;
+    const double bsum = block_sum<BS>(v, lds);
+    if(threadIdx.x == 0)
+    {
+        __hip_atomic_store(ra.partial + blockIdx.x, bsum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const int t = __hip_atomic_fetch_add(ra.ticket, 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+        last = t == (int)gridDim.x - 1;
+    }
+    __syncthreads();
+    if(!last) return;
+    double a = 0.0;
+    for(int i = threadIdx.x; i < (int)gridDim.x; i += BS)
+        a += __hip_atomic_load(ra.partial + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const double s = block_sum<BS>(a, lds);
+    if(threadIdx.x == 0)
+    {
+        apply_op(ra.op, s, ra.sc, ra.hist, ra.hist_cap, ra.out);
+        __hip_atomic_store(ra.ticket, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+}
+
+// phase 1, or both
+template <int BS>
+__device__ __forceinline__ void block_reduce(double v, const RedArgs& ra)
+{
+    if(ra.ticket)
+        block_total<BS>(v, ra);
+    else
+        block_partial<BS>(v, ra.partial, blockIdx.x);
+}
+
 // ---------------------------------------------------------------------------
 // Vector loads of R consecutive rows of one ELL slot.  A thread owns rows
 // [row, row+R) (row % R == 0, m % R == 0), so a wave issues one contiguous

@@ -157,7 +157,7 @@ __global__ __launch_bounds__(BS) void k_dot(int64_t n, const XT* __restrict__ x,
     chunk_range(n, b, e);
     double acc = 0.0;
     for(int64_t i = b + threadIdx.x; i < e; i += BS) acc = fmaT((double)y[i], (double)x[i], acc);
-    block_partial<BS>(acc, ra.partial, blockIdx.x);
+    block_reduce<BS>(acc, ra);
 }
 
 // w = alpha*x + beta*y with the reference's special cases (ComputeWAXPBY.cpp:63-91)
@@ -194,7 +194,7 @@ __global__ __launch_bounds__(BS) void k_axpy_dot(int64_t n, double alpha, const 
         y[i] = v;
         acc = fmaT(v, v, acc);
     }
-    block_partial<BS>(acc, ra.partial, blockIdx.x);
+    block_reduce<BS>(acc, ra);
 }
 
 // p = z (first iteration) or p = z + beta*p, with beta read on the device
@@ -243,7 +243,7 @@ __global__ __launch_bounds__(BS) void k_cg_xr(int64_t n, const double* __restric
         r[i] = rv;
         acc = fmaT(rv, rv, acc);
     }
-    block_partial<BS>(acc, ra.partial, blockIdx.x);
+    block_reduce<BS>(acc, ra);
 }
 
 // x += alpha*p if an iteration's x update is still pending (sc->xpend)
@@ -611,11 +611,33 @@ static unsigned red_grid(int64_t n)
 
 int64_t reduction_blocks(int64_t n) { return red_grid(n); }
 
-int launch_dot(int64_t n, const void* x, bool x_f64, const void* y, bool y_f64, const RedArgs& ra, hipStream_t s,
+// Reductions of at most this many blocks fold in the producer's last block
+// (block_total), the others in a launch of their own: the tickets of many blocks
+// queue at one address.  hpcgx_dot, one launch against two: 15.7 against 16.8 us
+// with 32 blocks (32^3), 16.0 against 16.4 with 63, 17.2 either way with 108 and
+// 20.1 against 17.2 with 256.
+constexpr unsigned ONE_LAUNCH_BLOCKS = 64;
+
+static_assert(ONE_LAUNCH_BLOCKS <= RED_THREADS, "block_total folds one partial a thread");
+
+static RedArgs one_launch(const RedArgs& ra, unsigned nblocks)
+{
+    RedArgs o = ra;
+    if(nblocks > ONE_LAUNCH_BLOCKS) o.ticket = nullptr;
+    return o;
+}
+
+static int end_reduction(unsigned nblocks, const RedArgs& ra, hipStream_t s, const int* gate)
+{
+    return ra.ticket ? 0 : launch_fold(nblocks, ra, s, gate);
+}
+
+int launch_dot(int64_t n, const void* x, bool x_f64, const void* y, bool y_f64, const RedArgs& rd, hipStream_t s,
                const int* gate)
 {
     constexpr int BS = RED_THREADS;
     const unsigned g = red_grid(n);
+    const RedArgs ra = one_launch(rd, g);
     if(x_f64 && y_f64)
         hipLaunchKernelGGL((k_dot<double, double, BS>), dim3(g), dim3(BS), 0, s, n, (const double*)x,
                            (const double*)y, ra, gate);
@@ -629,7 +651,7 @@ int launch_dot(int64_t n, const void* x, bool x_f64, const void* y, bool y_f64, 
         hipLaunchKernelGGL((k_dot<float, float, BS>), dim3(g), dim3(BS), 0, s, n, (const float*)x, (const float*)y,
                            ra, gate);
     HPCGX_KCHECK();
-    return launch_fold(g, ra, s, gate);
+    return end_reduction(g, ra, s, gate);
 }
 
 int launch_absdiff_max(int64_t n, const double* x, const double* y, double* partial, int64_t cap, double* out,
@@ -654,14 +676,15 @@ int launch_waxpby(int64_t n, double alpha, const double* x, double beta, const d
     return 0;
 }
 
-int launch_axpy_dot(int64_t n, double alpha, const double* x, double* y, const RedArgs& ra, hipStream_t s,
+int launch_axpy_dot(int64_t n, double alpha, const double* x, double* y, const RedArgs& rd, hipStream_t s,
                     const int* gate)
 {
     constexpr int BS = RED_THREADS;
     const unsigned g = red_grid(n);
+    const RedArgs ra = one_launch(rd, g);
     hipLaunchKernelGGL((k_axpy_dot<BS>), dim3(g), dim3(BS), 0, s, n, alpha, x, y, ra, gate);
     HPCGX_KCHECK();
-    return launch_fold(g, ra, s, gate);
+    return end_reduction(g, ra, s, gate);
 }
 
 int launch_cg_p(int64_t n, const void* z, bool z_f64, double* p, double* x, const CGScalars* sc, hipStream_t s,
@@ -678,13 +701,14 @@ int launch_cg_p(int64_t n, const void* z, bool z_f64, double* p, double* x, cons
     return 0;
 }
 
-int launch_cg_xr(int64_t n, const double* Ap, double* r, const RedArgs& ra, hipStream_t s, const int* gate)
+int launch_cg_xr(int64_t n, const double* Ap, double* r, const RedArgs& rd, hipStream_t s, const int* gate)
 {
     constexpr int BS = RED_THREADS;
     const unsigned g = red_grid(n);
+    const RedArgs ra = one_launch(rd, g);
     hipLaunchKernelGGL((k_cg_xr<BS>), dim3(g), dim3(BS), 0, s, n, Ap, r, ra, gate);
     HPCGX_KCHECK();
-    return launch_fold(g, ra, s, gate);
+    return end_reduction(g, ra, s, gate);
 }
 
 int launch_cg_xflush(int64_t n, const double* p, double* x, const CGScalars* sc, hipStream_t s, const int* gate)

@@ -26,6 +26,7 @@ struct RedArgs
     int hist_cap = -1;
     double* out = nullptr;
     int64_t cap = RED_BLOCKS;      // partial slots available
+    int* ticket = nullptr;         // blocks that have written their partial (0 between launches); null: fold launch
 };
 
 bool shape_supported(int rows, int block);

@@ -110,9 +110,15 @@ int problem_create(Problem*& out, int nx, int ny, int nz, int nlevels, bool with
     P->partial_cap = std::max<int64_t>(FOLD_MAX, (int64_t)(m0 / 64) + MAX_COLORS);
     if(alloc((void**)&P->sc, sizeof(CGScalars)) || alloc((void**)&P->hist, sizeof(double) * (P->hist_cap + 1)) ||
        alloc((void**)&P->partial, sizeof(double) * P->partial_cap) ||
-       alloc((void**)&P->dout, 8 * sizeof(double)))
+       alloc((void**)&P->dout, 8 * sizeof(double)) || alloc((void**)&P->ticket, sizeof(int)))
         return fail(-1);
-    if(hipMemsetAsync(P->sc, 0, sizeof(CGScalars), P->s) != hipSuccess)
+    if(hipHostMalloc((void**)&P->h_out, 8 * sizeof(double), hipHostMallocDefault) != hipSuccess)
+    {
+        set_error("hipHostMalloc failed");
+        return fail(-1);
+    }
+    if(hipMemsetAsync(P->sc, 0, sizeof(CGScalars), P->s) != hipSuccess ||
+       hipMemsetAsync(P->ticket, 0, sizeof(int), P->s) != hipSuccess)
         return fail(-1);
     if(coarse_build(*P)) return fail(-1);
     if(make_rhs(P->L[0], 0, 0, P->b, P->xexact, P->x, P->s)) return fail(-1);
@@ -165,6 +171,8 @@ void problem_destroy(Problem* P)
     f(P->hist);
     f(P->partial);
     f(P->dout);
+    f(P->ticket);
+    if(P->h_out) (void)hipHostFree(P->h_out);
     if(P->own_stream && P->s) (void)hipStreamDestroy(P->s);
     delete P;
 }
@@ -229,6 +237,7 @@ static RedArgs red(Problem& P, int op)
     ra.hist_cap = P.hist_cap;
     ra.out = P.dout;
     ra.cap = P.partial_cap;
+    ra.ticket = P.ticket;
     return ra;
 }
 

@@ -69,7 +69,8 @@ struct Problem
     int64_t partial_cap = 0;   // reduction partial slots
     double* dout = nullptr;   // OP_STORE results
     bool ext_cg = false;      // r/z64/p/Ap belong to the caller (drop-in CGData)
-    double h_out[8] = {};     // host landing slot of OP_STORE results
+    int* ticket = nullptr;    // of the reductions that take one launch (RedArgs::ticket)
+    double* h_out = nullptr;  // pinned, written by the kernels: results a call returns to the host
     CGScalars h_sc = {};      // host image of the scalars uploaded by cg_begin
 
     // CG run state
