@@ -150,6 +150,11 @@ struct Batch
     hipGraphExec_t gexec[2] = {nullptr, nullptr};
     int host_iter = 0;
     int mode = 0;
+    // every problem's CG scalars on the device, and where the host sees two
+    // iterations of them (pinned, written by kb_read_scalars; events tell when)
+    CGScalars** sc = nullptr;
+    CGScalars* h_sc = nullptr;
+    hipEvent_t read[2] = {nullptr, nullptr};
 };
 
 int batch_create(Batch*& B, int nprob, const int* dims, int nlevels, bool with_f64, bool with_mixed, hipStream_t s);
