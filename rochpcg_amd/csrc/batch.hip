@@ -334,12 +334,14 @@ struct Planner
         return l;
     }
 
-    int block(int l)
+    int64_t level_rows(int l)
     {
         int64_t m = 0;
         for(const Problem* P : B.probs) m += P->L[l].m;
-        return B.block[l] ? B.block[l] : default_block(m);
+        return m;
     }
+
+    int block(int l) { return B.block[l] ? B.block[l] : default_block(level_rows(l)); }
 
     int max_colors(int l)
     {
@@ -473,6 +475,10 @@ struct Planner
     int outer_spmv(bool dot, bool from_x, bool into_tmp)
     {
         next_subs = max_colors(0);   // one segment per colour: a block stages one colour's patterns
+        // two rows a thread where one problem of as many rows has them
+        // (default_shapes): 64 problems of 12.5M rows take 576 us in place of 645 in
+        // FP64, 275 in place of 331 mixed
+        next_rows = level_rows(0) > SMALL_ROWS ? 2 : 1;
         return add(BK_SPMV, block(0), false, 1, dot ? 1 : 0, 0.0, [&](int k, BSeg& s) {
             Problem* P = B.probs[k];
             const Level& L = P->L[0];

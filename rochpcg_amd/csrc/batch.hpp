@@ -81,7 +81,7 @@ inline int64_t assign_blocks(BSeg* segs, size_t nseg, int block, bool vector_kin
     return nb;
 }
 
-// Rows per thread a sweep launch can use: 2 loads R consecutive rows of a
+// Rows per thread a launch can use: 2 loads R consecutive rows of a
 // slot as one vector, which needs even offsets and sizes in every segment
 // (an even row's pair then shares its ELL slice); otherwise 1.
 inline int launch_rows(const BSeg* segs, size_t nseg, int rows)
@@ -120,7 +120,7 @@ struct BLaunch
     int win;          // sweeps: widest slot window of the launch's segments (Level::win)
     int win_tail;     // post-smoother forward sweep: widest last-colour window
     int all_u;        // post-smoother forward sweep: every segment reuses its upper sums
-    int rows;         // sweeps: rows per thread (1 or 2)
+    int rows;         // SpMV, sweeps: rows per thread (1 or 2)
     int pat;          // row kernels: every segment has row patterns
     int nseg;
     int64_t nblocks;

@@ -15,18 +15,24 @@ namespace hpcgx
     Cols<PAT, (R), BS> cols(S.cols, pat_lds, row, true);
 
 // the whole level, block by block of one colour (one segment per colour)
-template <bool PAT, typename VT, typename XT, typename YT, bool DOT, int BS>
+template <bool PAT, typename VT, typename XT, typename YT, bool DOT, int R, int BS>
 __global__ __launch_bounds__(BS) void kb_spmv(const BSeg* __restrict__ segs, int nseg)
 {
     BSEG();
-    BCOLS(1);
+    BCOLS(R);
     double acc = 0.0;
-    XT s[1];
-    row_spmv<VT, XT, 1>(row, cols, (const VT*)S.val, (const XT*)S.r, s);
+    XT s[R];
+    row_spmv<VT, XT, R>(row, cols, (const VT*)S.val, (const XT*)S.r, s);
     if(live)
     {
-        ((YT*)S.x)[row] = (YT)s[0];
-        if(DOT) acc = fmaT((double)((const XT*)S.r)[row], (double)s[0], acc);
+        st_cvt<R>((YT*)S.x + row, s);
+        if(DOT)
+        {
+            XT xr[R];
+            ld<R>((const XT*)S.r + row, xr);
+#pragma unroll
+            for(int k = 0; k < R; ++k) acc = fmaT((double)xr[k], (double)s[k], acc);
+        }
     }
     if(DOT) block_partial<BS>(acc, S.ra.partial, S.part0 + lb);
 }
@@ -118,20 +124,23 @@ static void launch_rows_bs(const BLaunch& L, hipStream_t s)
     {
     case BK_SPMV:
         // outer SpMV: f64 vectors over either store; MG-internal SpMV is not batched
-        if(f64)
-        {
-            if(L.dot)
-                hipLaunchKernelGGL((kb_spmv<PAT, double, double, double, true, BS>), g, b, 0, s, T, n);
+        with_rows(L.rows, [&](auto RR) {
+            constexpr int R = decltype(RR)::value;
+            if(f64)
+            {
+                if(L.dot)
+                    hipLaunchKernelGGL((kb_spmv<PAT, double, double, double, true, R, BS>), g, b, 0, s, T, n);
+                else
+                    hipLaunchKernelGGL((kb_spmv<PAT, double, double, double, false, R, BS>), g, b, 0, s, T, n);
+            }
             else
-                hipLaunchKernelGGL((kb_spmv<PAT, double, double, double, false, BS>), g, b, 0, s, T, n);
-        }
-        else
-        {
-            if(L.dot)
-                hipLaunchKernelGGL((kb_spmv<PAT, __half, double, double, true, BS>), g, b, 0, s, T, n);
-            else
-                hipLaunchKernelGGL((kb_spmv<PAT, __half, double, double, false, BS>), g, b, 0, s, T, n);
-        }
+            {
+                if(L.dot)
+                    hipLaunchKernelGGL((kb_spmv<PAT, __half, double, double, true, R, BS>), g, b, 0, s, T, n);
+                else
+                    hipLaunchKernelGGL((kb_spmv<PAT, __half, double, double, false, R, BS>), g, b, 0, s, T, n);
+            }
+        });
         break;
     case BK_FWD_ZERO:
         with_rows(L.rows, [&](auto RR) {
