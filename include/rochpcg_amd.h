@@ -83,7 +83,10 @@ int hpcgx_color_table(const hpcgx_problem* p, int level, int* sizes, int* offset
  * natural -> coarse multicolour row), row descriptors (int32: diagonal slot
  * in bits 0-7, first slot of an off-diagonal last-colour column in bits 8-15,
  * first upper slot in bits 16-23, 27 when absent; no reference counterpart), diagonal
- * values f64 (or NULL) and f16 (or NULL) (no reference counterpart) */
+ * values f64 (or NULL) and f16 (or NULL) (no reference counterpart).  The
+ * kernels read the columns from copies made with the problem (row patterns,
+ * and the coarse levels' own), so columns and descriptors written through these
+ * pointers are not followed; values and diagonals are read where they lie */
 int hpcgx_level_arrays(const hpcgx_problem* p, int level, void** ptrs);
 /* device pointers of the CG data and system: ptrs[0..7] = b, x, xexact, r,
  * z (f64, or NULL), p, Ap, z (f32 mixed-mode, or NULL)  (CGData.hpp:55-61) */

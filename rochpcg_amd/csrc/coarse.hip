@@ -438,6 +438,7 @@ static int build_plan(Problem& P, Prec prec)
     const size_t step_at = 2 * ncol, lv_at = step_at + sizeof(CoarseStep) * steps.size();
     const size_t bytes = lv_at + sizeof(CoarseLevel) * nc;
     HPCGX_HIP(hipMalloc(&C.mem, bytes));
+    C.bytes = bytes;
     char* mem = (char*)C.mem;
     for(int j = 0; j < nc; ++j)
     {

@@ -149,7 +149,7 @@ struct Level
     // row patterns (null: the rows repeat too little, or the level is too
     // large for 32-bit gather offsets); derived from ell_col and desc
     uint8_t* pat = nullptr;       // [m] pattern of each row, within its colour
-    int32_t* pat_tab = nullptr;   // [ncolors][PAT_MAX][PAT_QUADS*4]
+    int32_t* pat_tab = nullptr;   // [ncolors][PAT_MAX][PAT_QUADS*4], in the allocation of pat
     int npat = 0;                 // patterns of the colour that has most
     bool pat_off = false;         // the kernels read the column array all the same
     double* inv_diag = nullptr;   // [m] 1/a_ii (f64)

@@ -3,9 +3,10 @@
 //
 // All operators are HBM-bound sparse/streaming work: one thread per row,
 // sliced ELL (entry p of row r at ell_at(p, r), common.hpp) so every slot load
-// of a wave is one contiguous 256 B (cols) / 512 B (f64 values) segment and
-// the slots of a slice follow each other, matrix streams loaded non-temporally, x gathered through L2/MALL.  Row tiles are laid out
-// so each XCD works on one contiguous spatial slab (xcd_block), which keeps
+// of a wave is one contiguous segment (512 B of f64 values) and the slots of a
+// slice follow each other, values loaded non-temporally, columns from the row
+// patterns (Cols in kernels.hpp), x gathered through L2/MALL.  Row tiles are laid
+// out so each XCD works on one contiguous spatial slab (xcd_block), which keeps
 // the neighbours a slab gathers inside that XCD's L2.
 //
 // Reference kernels whose results these reproduce:

@@ -581,6 +581,7 @@ int64_t problem_device_bytes(const Problem& P)
     }
     const int64_t m0 = P.L[0].m;
     b += 7 * 8 * m0 + (P.has_f64 ? 8 * m0 : 0) + (P.has_mixed ? 4 * m0 : 0);   // CG vectors, z
+    for(const CoarsePlan& C : P.coarse) b += (int64_t)C.bytes;
     b += 8 * P.partial_cap + 8 * (P.hist_cap + 1) + (int64_t)sizeof(CGScalars) + 64;
     return b;
 }

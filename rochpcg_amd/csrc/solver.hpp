@@ -38,6 +38,7 @@ struct CoarsePlan
 {
     int first = MAX_LEVELS;        // first level that can run so
     void* mem = nullptr;           // descriptions, steps and columns
+    size_t bytes = 0;              // of mem
     CoarseLevel* lv = nullptr;     // of level `first`
     size_t lds[MAX_LEVELS] = {};   // LDS of a run from each level
 };
