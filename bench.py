@@ -9,7 +9,7 @@ configuration, about 70 GB of HBM), all arrays resident in HBM.
 Prints one JSON line: the FP64 HPCG-formula GFLOP/s (value), the mixed-
 precision CG's GFLOP/s (f64 true residual every 10 iterations) and both
 solves' time to a relative residual of 1e-9 (x* from splitmix64 seed 99), the
-modelled HBM TB/s, a roofline entry for the outer SpMV kernel timed with HIP
+modelled HBM TB/s (bytes the kernels load and store), a roofline entry for the outer SpMV kernel timed with HIP
 events on the solver stream, a second leg at 320^3 (seed 1234), the
 64-problem batched leg, and the CPU baseline (the reference's own CG_ref,
 OpenMP, on this host's cores, on a bounded sample).
@@ -46,6 +46,24 @@ def profiled_traffic(dims):
 
 def spmv_bytes(m, vb=8):
     return m * (27 * (4 + vb) + 8 + 8)
+
+
+def spmv_loaded_bytes(m, vb=8):
+    """What the SpMV loads where the level has row patterns: the values, one byte
+    a row for its columns, x and y (spmv_bytes counts the ELL's 4 B column a slot)."""
+    return m * (27 * vb + 1 + 8 + 8)
+
+
+def loaded_traffic(dims):
+    """profiled_traffic of the kernel that reads row patterns, or None."""
+    import re
+    path = os.path.join(ROOT, "profiles", f"row_patterns_{dims[0]}x{dims[1]}x{dims[2]}.md")
+    try:
+        with open(path) as f:
+            found = re.search(r"^k_spmv f64, HBM bytes per launch: (\d+)", f.read(), re.M)
+            return int(found.group(1)) if found else None
+    except OSError:
+        return None
 
 
 def vcycle_compulsory_bytes(level_rows):
@@ -127,17 +145,19 @@ def batched_leg(hip, count, log):
             P.vec["x"].upload(np.zeros(P.m))
         prof = B.profile(iters=5, mode=mode)
         it_ms, it_bytes = prof.pop("iteration")
-        kinds = {k: {"ms": round(ms, 4), "GBps": round(by / (ms * 1e-3) / 1e9, 1) if ms > 0 else None}
+        # per kind by the ELL's bytes (4 B column a slot); the iteration also by what
+        # its kernels load and store
+        kinds = {k: {"ms": round(ms, 4), "ell_GBps": round(by / (ms * 1e-3) / 1e9, 1) if ms > 0 else None}
                  for k, (ms, by) in prof.items() if by > 0}
-        dom = max(prof, key=lambda k: prof[k][0])
-        dms, dby = prof[dom]
+        loaded = sum(P.stream_bytes(mode)[1] for P in B.problems)
+        gbps = loaded / (it_ms * 1e-3) / 1e9
         res[f"roofline_{name}"] = {
-            "kernel": f"batched {dom} launches (all levels and colours, one launch per colour for all problems)",
-            "bound": "hbm", "achieved": round(dby / (dms * 1e-3) / 1e9, 1), "peak": HBM_PEAK_GBPS,
-            "unit": "GB/s", "frac": round(dby / (dms * 1e-3) / 1e9 / HBM_PEAK_GBPS, 4),
-            "bytes_per_iteration": int(dby), "ms_per_iteration": round(dms, 4),
-            "iteration_ms": round(it_ms, 4), "iteration_GBps": round(it_bytes / (it_ms * 1e-3) / 1e9, 1),
-            "kinds": kinds}
+            "kernel": "one batched iteration, eager launches (all levels and colours, one launch per colour for "
+                      "all problems)",
+            "bound": "hbm", "achieved": round(gbps, 1), "peak": HBM_PEAK_GBPS,
+            "unit": "GB/s", "frac": round(gbps / HBM_PEAK_GBPS, 4),
+            "bytes_per_iteration": int(loaded), "ell_bytes_per_iteration": int(it_bytes),
+            "iteration_ms": round(it_ms, 4), "kinds": kinds}
         log(f"batched {name} profile: {res[f'roofline_{name}']}")
     B.close()
     return res
@@ -279,10 +299,13 @@ def main():
     G.set_residual_replacement(0)
     log(f"mixed, true residual every 10: {K} iterations in {elmr * 1e3:.1f} ms")
     ms64, msmx, msmr = (e * 1e3 / K for e in (el64, elmx, elmr))
-    # algorithmic bytes of this library's kernels (each ELL slot a kernel reads
-    # once, neighbour gathers from cache, own-row vectors once)
-    mg64, b64 = G.iteration_bytes(hip.CG_F64)
-    _, bmx = G.iteration_bytes(hip.CG_MIXED)
+    # bytes this library's kernels load and store (each slot a kernel reads once: its
+    # value, the columns as one byte a row; neighbour gathers from cache, own-row
+    # vectors once), and the same with the ELL's 4 B column a slot
+    mg64, b64 = G.stream_bytes(hip.CG_F64)
+    _, bmx = G.stream_bytes(hip.CG_MIXED)
+    _, ell64 = G.iteration_bytes(hip.CG_F64)
+    _, ellmx = G.iteration_bytes(hip.CG_MIXED)
 
     # per-phase HIP-event timing of K FP64 iterations (eager launches)
     G.vec["x"].upload(np.zeros(G.m))
@@ -290,7 +313,7 @@ def main():
     ph = G.cg_iterate_profiled(K)
     G.cg_end()
     spmv_ms = ph["spmv"] / K
-    spmv_gbps = spmv_bytes(G.m) / (spmv_ms * 1e-3) / 1e9
+    spmv_gbps = spmv_loaded_bytes(G.m) / (spmv_ms * 1e-3) / 1e9
     mg_ms = ph["mg"] / K
     mg_gbps = mg64 / (mg_ms * 1e-3) / 1e9
     # the same time against the full-row compulsory byte model (the sweeps here
@@ -304,7 +327,7 @@ def main():
     ceil64 = 27 * 12 * me / (G.time_operator(hip.OP_READ_STREAM, 0, mixed=False, reps=10) * 1e-3) / 1e9
     ceil16 = 27 * 6 * me / (G.time_operator(hip.OP_READ_STREAM, 0, mixed=True, reps=10) * 1e-3) / 1e9
     spmv16_ms = G.time_operator(hip.OP_SPMV, 0, mixed=True, reps=K)
-    spmv16_gbps = spmv_bytes(G.m, 2) / (spmv16_ms * 1e-3) / 1e9
+    spmv16_gbps = spmv_loaded_bytes(G.m, 2) / (spmv16_ms * 1e-3) / 1e9
     log(f"read ceiling of the matrix stream: {ceil64:.0f} GB/s (f64 values), {ceil16:.0f} GB/s (f16 values); "
         f"mixed SpMV {spmv16_ms:.3f} ms, {spmv16_gbps:.0f} GB/s")
 
@@ -329,24 +352,26 @@ def main():
                    "graph": use_graph, "parallelism": "single GPU", "level0_shapes": tuned},
         "setup_s": round(setup_s, 3),
         "hbm_TBps": round(b64 / (ms64 * 1e-3) / 1e12, 3),
-        "bytes_per_iteration": int(b64),
+        "bytes_per_iteration": int(b64), "ell_bytes_per_iteration": int(ell64),
         "mixed": {"value": round(flops / (msmr * 1e-3) / 1e9, 2), "unit": "GFLOP/s",
                   "ms_per_step": round(msmr, 4), "true_residual_every": 10,
                   "ms_per_step_no_refinement": round(msmx, 4),
                   "hbm_TBps": round(bmx / (msmx * 1e-3) / 1e12, 3),
-                  "bytes_per_iteration": int(bmx), "speedup_per_iteration": round(ms64 / msmr, 3),
+                  "bytes_per_iteration": int(bmx), "ell_bytes_per_iteration": int(ellmx), "speedup_per_iteration": round(ms64 / msmr, 3),
                   "dtype": "f64 outer CG / f32 vectors + f16 ELL in MG"},
         "phase_ms_per_iteration": {k: round(v / K, 4) for k, v in ph.items()},
         "roofline": {"kernel": "k_spmv (outer SpMV + fused p'Ap), level 0",
                      "bound": "hbm", "achieved": round(spmv_gbps, 1), "peak": HBM_PEAK_GBPS,
                      "unit": "GB/s", "frac": round(spmv_gbps / HBM_PEAK_GBPS, 4),
-                     "traffic": profiled_traffic(dims), "bytes_per_launch": spmv_bytes(G.m),
+                     "traffic": loaded_traffic(dims), "bytes_per_launch": spmv_loaded_bytes(G.m),
+                     "ell_bytes_per_launch": spmv_bytes(G.m),
                      "avg_launch_ms": round(spmv_ms, 4),
                      "read_ceiling_GBps": round(ceil64, 1), "frac_of_read_ceiling": round(spmv_gbps / ceil64, 4)},
         "mixed_spmv_roofline": {"kernel": "k_spmv (f16 values, f64 vectors, fused p'Ap), level 0",
                                 "bound": "hbm", "achieved": round(spmv16_gbps, 1), "peak": HBM_PEAK_GBPS,
                                 "unit": "GB/s", "frac": round(spmv16_gbps / HBM_PEAK_GBPS, 4),
-                                "bytes_per_launch": spmv_bytes(G.m, 2), "avg_launch_ms": round(spmv16_ms, 4),
+                                "bytes_per_launch": spmv_loaded_bytes(G.m, 2),
+                                "ell_bytes_per_launch": spmv_bytes(G.m, 2), "avg_launch_ms": round(spmv16_ms, 4),
                                 "read_ceiling_GBps": round(ceil16, 1),
                                 "frac_of_read_ceiling": round(spmv16_gbps / ceil16, 4)},
         "mg_roofline": {"kernels": "FP64 V-cycle, all levels (sweeps, restriction, prolongation)",
