@@ -289,7 +289,7 @@ struct Planner
             std::memcpy(h.data(), segs.data(), sizeof(BSeg) * segs.size());
             block_map(segs.data(), segs.size(), reinterpret_cast<uint16_t*>(h.data() + sizeof(BSeg) * segs.size()));
             BSeg* d = nullptr;
-            HPCGX_HIP(hipMalloc(&d, h.size()));
+            HPCGX_HIP(hipMalloc(&d, h.size() + 2));   // seg_of reads whole words of the map
             B.tables.push_back(d);
             HPCGX_HIP(hipMemcpy(d, h.data(), h.size(), hipMemcpyHostToDevice));
             L.segs = d;

@@ -22,7 +22,11 @@ __device__ __forceinline__ T cvt(float v) { return (T)v; }
 template <typename T>
 __device__ __forceinline__ T cvt(__half v) { return (T)__half2float(v); }
 
-__device__ __forceinline__ bool gated(const int* gate) { return gate != nullptr && *gate != 0; }
+__device__ __forceinline__ bool gated(const int* gate)
+{
+    typedef const __attribute__((address_space(4))) int ConstInt;   // an earlier launch wrote it: a scalar load
+    return gate != nullptr && *(ConstInt*)gate != 0;
+}
 
 // ---------------------------------------------------------------------------
 // deterministic two-phase reductions (block partials, then one fold block);
