@@ -19,8 +19,9 @@ __device__ __forceinline__ int seg_of(const BSeg* segs, int nseg, int64_t b)
 // A block's way to its rows: map -> segment -> flag -> pattern, each a load that
 // waits for the one before.  All are scalar loads, and the fields every kernel needs
 // come together (the asm has them in registers before the flag is looked at); with
-// vector loads of the map and the flag and the fields behind the flag, 20 iterations
-// of 64 problems took 61.0 and 33.2 ms (FP64, mixed) where they take 58.5 and 30.0.
+// vector loads of the map and the flag and the fields behind the flag, 64 problems of
+// 16^3 to 96^3 took 131.7 and 72.9 ms to 1e-9 (FP64, mixed) where they take 128.4 and
+// 68.6.
 #define BSEG()                                                                                              \
     const int64_t b_ = xcd_block(blockIdx.x, gridDim.x);                                                    \
     const BSeg& S = segs[seg_of(segs, nseg, b_)];                                                           \
