@@ -20,8 +20,12 @@ namespace hpcgx
 // reversed launch): each XCD then starts a launch on the slab it finished the
 // previous one on, whose neighbours' x is still in its caches.  Threads past
 // the end work on the last rows and store nothing.
+// The flag that stops converged solves is looked at behind the row's arithmetic
+// and its pattern's load (cheap, and in range whatever the flag), ahead of its
+// values: an iteration of 104^3 takes 553 in place of 569 us in FP64 and 397 in
+// place of 412 mixed, one that is stopped the same 0.17 ms.
 #define SWEEP_ROW()                                                                   \
-    if(gated(gate)) return;                                                           \
+    const bool stop_ = gated(gate);                                                   \
     PAT_LDS();                                                                        \
     int64_t Lb_ = xcd_block(blockIdx.x, gridDim.x);                                   \
     if(size < 0)                                                                      \
@@ -39,7 +43,8 @@ namespace hpcgx
     const int64_t i = Lb_ * (BS * R) + (int64_t)threadIdx.x * R;                      \
     const bool live = i < size;                                                       \
     const int64_t row = off + (live ? i : size - R);                                  \
-    Cols<PAT, R, BS> cols(ca, pat_lds, row, true);
+    Cols<PAT, R, BS> cols(ca, pat_lds, row, true);                                    \
+    if(stop_) return;
 
 template <bool PAT, int NS, typename VT, typename XT, typename RT, int R, int BS>
 __global__ __launch_bounds__(BS) void k_fwd_zero(int64_t off, int64_t size, ZMap zm, ColArgs ca, const VT* __restrict__ val,
