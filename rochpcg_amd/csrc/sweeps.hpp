@@ -23,7 +23,8 @@ namespace hpcgx
 // The flag that stops converged solves is looked at behind the row's arithmetic
 // and its pattern's load (cheap, and in range whatever the flag), ahead of its
 // values: an iteration of 104^3 takes 553 in place of 569 us in FP64 and 397 in
-// place of 412 mixed, one that is stopped the same 0.17 ms.
+// place of 412 mixed, one that is stopped the same 0.17 ms.  The kernels take the
+// flag and what the row's arithmetic needs first, where arguments are preloaded.
 #define SWEEP_ROW()                                                                   \
     const bool stop_ = gated(gate);                                                   \
     PAT_LDS();                                                                        \
@@ -47,18 +48,18 @@ namespace hpcgx
     if(stop_) return;
 
 template <bool PAT, int NS, typename VT, typename XT, typename RT, int R, int BS>
-__global__ __launch_bounds__(BS) void k_fwd_zero(int64_t off, int64_t size, ZMap zm, ColArgs ca, const VT* __restrict__ val,
+__global__ __launch_bounds__(BS) void k_fwd_zero(const int* gate, int64_t off, int64_t size, const VT* __restrict__ val,
                                                  const VT* __restrict__ dg, const RT* __restrict__ r,
-                                                 XT* __restrict__ x, const int* gate)
+                                                 XT* __restrict__ x, ZMap zm, ColArgs ca)
 {
     SWEEP_ROW();
     row_fwd_zero<NS, VT, XT, RT, R>(row, live, cols, val, dg, r, x);
 }
 
 template <bool PAT, int NS, typename VT, typename XT, bool STORE_U, int R, int BS>
-__global__ __launch_bounds__(BS) void k_bwd_zero(int64_t off, int64_t size, ZMap zm, ColArgs ca, const VT* __restrict__ val,
+__global__ __launch_bounds__(BS) void k_bwd_zero(const int* gate, int64_t off, int64_t size, const VT* __restrict__ val,
                                                  const VT* __restrict__ dg, XT* __restrict__ x, XT* __restrict__ u,
-                                                 const int* gate)
+                                                 ZMap zm, ColArgs ca)
 {
     SWEEP_ROW();
     row_bwd_zero<NS, VT, XT, STORE_U, R>(row, live, cols, val, dg, x, u);
@@ -74,19 +75,19 @@ __global__ __launch_bounds__(BS) void k_fwd_full(int64_t off, int64_t size, ZMap
 }
 
 template <bool PAT, int NA, int NB, typename VT, typename XT, typename RT, int R, int BS>
-__global__ __launch_bounds__(BS) void k_fwd_full_u(int64_t off, int64_t size, ZMap zm, ColArgs ca,
+__global__ __launch_bounds__(BS) void k_fwd_full_u(const int* gate, int64_t off, int64_t size,
                                                    const VT* __restrict__ val, const VT* __restrict__ dg,
                                                    const RT* __restrict__ r, XT* __restrict__ x, XT* __restrict__ t,
-                                                   const int* gate)
+                                                   ZMap zm, ColArgs ca)
 {
     SWEEP_ROW();
     row_fwd_full_u<NA, NB, VT, XT, RT, R>(row, live, cols, val, dg, r, x, t);
 }
 
 template <bool PAT, int NS, typename VT, typename XT, int R, int BS>
-__global__ __launch_bounds__(BS) void k_bwd_full(int64_t off, int64_t size, ZMap zm, ColArgs ca, const VT* __restrict__ val,
+__global__ __launch_bounds__(BS) void k_bwd_full(const int* gate, int64_t off, int64_t size, const VT* __restrict__ val,
                                                  const VT* __restrict__ dg, const XT* __restrict__ t,
-                                                 XT* __restrict__ x, const int* gate)
+                                                 XT* __restrict__ x, ZMap zm, ColArgs ca)
 {
     SWEEP_ROW();
     row_bwd_full<NS, VT, XT, R>(row, live, cols, val, dg, t, x);
@@ -166,8 +167,8 @@ static int sweep_t(const Level& L, int part, const void* rv, void* xv, void* tv,
         constexpr int R = decltype(RR)::value, BS = decltype(BB)::value;
         with_window(L.win[WIN_LOWER][c], [&](auto NN) {
             constexpr int NS = decltype(NN)::value;
-            hipLaunchKernelGGL((k_fwd_zero<PAT, NS, VT, XT, RT, R, BS>), grid, dim3(BS), 0, s, (int64_t)L.offsets[c],
-                               sz, zm, L.cols(c), val, dg, r, x, gate);
+            hipLaunchKernelGGL((k_fwd_zero<PAT, NS, VT, XT, RT, R, BS>), grid, dim3(BS), 0, s, gate,
+                               (int64_t)L.offsets[c], sz, val, dg, r, x, zm, L.cols(c));
         });
     };
     switch(part)
@@ -182,10 +183,10 @@ static int sweep_t(const Level& L, int part, const void* rv, void* xv, void* tv,
                 constexpr int NS = decltype(NN)::value;
                 if(part == 4)
                     hipLaunchKernelGGL((k_bwd_zero<PAT, NS, VT, XT, true, R, BS>), grid, dim3(BS), 0, s,
-                                       (int64_t)L.offsets[c], sz, zm, L.cols(c), val, dg, x, t, gate);
+                                       gate, (int64_t)L.offsets[c], sz, val, dg, x, t, zm, L.cols(c));
                 else
                     hipLaunchKernelGGL((k_bwd_zero<PAT, NS, VT, XT, false, R, BS>), grid, dim3(BS), 0, s,
-                                       (int64_t)L.offsets[c], sz, zm, L.cols(c), val, dg, x, t, gate);
+                                       gate, (int64_t)L.offsets[c], sz, val, dg, x, t, zm, L.cols(c));
             });
         });
     case 2:
@@ -198,7 +199,7 @@ static int sweep_t(const Level& L, int part, const void* rv, void* xv, void* tv,
                 with_window_pair(L.win[WIN_LOWER][c], L.win[WIN_TAIL][c], [&](auto NA_, auto NB_) {
                     constexpr int NA = decltype(NA_)::value, NB = decltype(NB_)::value;
                     hipLaunchKernelGGL((k_fwd_full_u<PAT, NA, NB, VT, XT, RT, R, BS>), grid, dim3(BS), 0, s,
-                                       (int64_t)L.offsets[c], sz, zm, L.cols(c), val, dg, r, x, t, gate);
+                                       gate, (int64_t)L.offsets[c], sz, val, dg, r, x, t, zm, L.cols(c));
                 });
             else
                 hipLaunchKernelGGL((k_fwd_full<PAT, VT, XT, RT, R, BS>), grid, dim3(BS), 0, s,
@@ -211,7 +212,7 @@ static int sweep_t(const Level& L, int part, const void* rv, void* xv, void* tv,
             with_window(L.win[WIN_UPPER][c], [&](auto NN) {
                 constexpr int NS = decltype(NN)::value;
                 hipLaunchKernelGGL((k_bwd_full<PAT, NS, VT, XT, R, BS>), grid, dim3(BS), 0, s,
-                                   (int64_t)L.offsets[c], sz, zm, L.cols(c), val, dg, (const XT*)t, x, gate);
+                                   gate, (int64_t)L.offsets[c], sz, val, dg, (const XT*)t, x, zm, L.cols(c));
             });
         });
     }
