@@ -15,8 +15,8 @@
 // slot, without masks or selects; the rest is a division and a barrier.
 //
 // Measured, a CG iteration of FP64 / mixed with every level as launches and with
-// its coarse levels here: 16^3 307 / 262 -> 149 / 115 us, 32^3 361 / 289 ->
-// 246 / 186 us, 64^3 466 / 352 -> 408 / 285 us, 104^3 668 / 473 -> 641 / 442 us;
+// its coarse levels here: 16^3 254 / 238 -> 148 / 114 us, 32^3 282 / 254 ->
+// 220 / 171 us, 64^3 382 / 313 -> 358 / 268 us, 104^3 561 / 418 -> 545 / 391 us;
 // a step takes 0.5-0.9 us.
 //
 // Per row the arithmetic is that of the row_* functions of kernels.hpp, slot by

@@ -43,10 +43,11 @@ struct CoarsePlan
     size_t lds[MAX_LEVELS] = {};   // LDS of a run from each level
 };
 // Levels of at most this many rows run so, [precision].  One workgroup streams a
-// level's values at one CU's rate, launches at the GPU's: at 4096 rows it takes
-// 16 us less for the coarsest level of an FP64 V-cycle and 21 us less for that
-// of a mixed one, at 5832 rows 9 us more and 16 us less, at 8000 rows 66 us more
-// and 5 us less (the f16 values are a quarter of the bytes).
+// level's values at one CU's rate, launches at the GPU's: an iteration of 64^3,
+// whose third level has 4096 rows, takes 24 us less in FP64 and 45 less mixed with
+// it and the level below in one; the third level of 72^3, 5832 rows, costs 30 us
+// more and saves 13, that of 80^3, 8000 rows, costs 91 and 2 (the f16 values are a
+// quarter of the bytes).
 constexpr int COARSE_ROWS[2] = {5000, 8191};
 
 struct Problem
