@@ -53,7 +53,8 @@ Context& ctx()
     {
         if(hipGetDevice(&c.device) != hipSuccess || hipStreamCreateWithFlags(&c.s, hipStreamNonBlocking) != hipSuccess ||
            hipMalloc(&c.partial, sizeof(double) * FOLD_MAX) != hipSuccess ||
-           hipMalloc(&c.ticket, sizeof(int)) != hipSuccess || hipMemset(c.ticket, 0, sizeof(int)) != hipSuccess ||
+           hipMalloc(&c.ticket, sizeof(int)) != hipSuccess ||
+           hipMemsetAsync(c.ticket, 0, sizeof(int), c.s) != hipSuccess ||
            hipHostMalloc((void**)&c.h_out, sizeof(double), hipHostMallocDefault) != hipSuccess)
         {
             fprintf(stderr, "rochpcg_amd: cannot initialise the HIP context\n");
