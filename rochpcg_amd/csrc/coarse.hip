@@ -434,11 +434,10 @@ static int build_plan(Problem& P, Prec prec)
     }
     const int nc = nl - C.first;
     if(nc == 0) return 0;
-    // one allocation: columns (a multiple of 8 bytes), steps, descriptions
-    const size_t step_at = 2 * ncol, lv_at = step_at + sizeof(CoarseStep) * steps.size();
-    const size_t bytes = lv_at + sizeof(CoarseLevel) * nc;
-    HPCGX_HIP(hipMalloc(&C.mem, bytes));
-    C.bytes = bytes;
+    // one allocation: columns, steps, descriptions
+    const CoarseLayout lay = coarse_layout(ncol, steps.size(), nc);
+    HPCGX_HIP(hipMalloc(&C.mem, lay.bytes));
+    C.bytes = lay.bytes;
     char* mem = (char*)C.mem;
     for(int j = 0; j < nc; ++j)
     {
@@ -450,7 +449,7 @@ static int build_plan(Problem& P, Prec prec)
         h[j].at = (const uint2*)((uint16_t*)mem + cols[j]);
         h[j].f2c_fine = L.f2c_fine;
         h[j].f2c_coarse = L.f2c_coarse;
-        h[j].steps = (const CoarseStep*)(mem + step_at) + first_step[j];
+        h[j].steps = (const CoarseStep*)(mem + lay.steps) + first_step[j];
         h[j].r = V.r;
         h[j].x = V.x;
         h[j].m = (int)L.m;
@@ -459,12 +458,12 @@ static int build_plan(Problem& P, Prec prec)
                            prec == PREC_F64 ? 8 : 4, L.ell_col, L.desc, (uint16_t*)mem + cols[j]);
         HPCGX_HIP(hipGetLastError());
     }
-    std::vector<char> up(bytes - step_at);
+    std::vector<char> up(lay.bytes - lay.steps);
     std::memcpy(up.data(), steps.data(), sizeof(CoarseStep) * steps.size());
-    std::memcpy(up.data() + (lv_at - step_at), h.data(), sizeof(CoarseLevel) * nc);
-    HPCGX_HIP(hipMemcpyAsync(mem + step_at, up.data(), up.size(), hipMemcpyHostToDevice, P.s));
+    std::memcpy(up.data() + (lay.levels - lay.steps), h.data(), sizeof(CoarseLevel) * nc);
+    HPCGX_HIP(hipMemcpyAsync(mem + lay.steps, up.data(), up.size(), hipMemcpyHostToDevice, P.s));
     HPCGX_HIP(hipStreamSynchronize(P.s));
-    C.lv = (CoarseLevel*)(mem + lv_at);
+    C.lv = (CoarseLevel*)(mem + lay.levels);
     return 0;
 }
 

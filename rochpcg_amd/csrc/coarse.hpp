@@ -53,6 +53,24 @@ struct CoarseRun
     const int* gate;
 };
 
+// Where the parts of a plan's allocation lie, in bytes: the columns, from 0, then
+// the steps, then the descriptions, which hold pointers and start where those may
+// (the bottom of an eight-colour hierarchy has 15 steps of 36 bytes).
+struct CoarseLayout
+{
+    size_t steps, levels, bytes;
+};
+
+inline CoarseLayout coarse_layout(size_t ncolumns, size_t nsteps, size_t nlevels)
+{
+    auto up = [](size_t at, size_t a) { return (at + a - 1) / a * a; };
+    CoarseLayout o;
+    o.steps = up(sizeof(uint16_t) * ncolumns, alignof(CoarseStep));
+    o.levels = up(o.steps + sizeof(CoarseStep) * nsteps, alignof(CoarseLevel));
+    o.bytes = o.levels + sizeof(CoarseLevel) * nlevels;
+    return o;
+}
+
 // build the plans of a problem whose levels and vectors exist
 int coarse_build(Problem& P);
 void coarse_free(Problem& P);
