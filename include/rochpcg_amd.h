@@ -240,7 +240,7 @@ int hpcgx_cg_ref(hpcgx_problem* p, const double* b, double* x, int max_iter, dou
  * (dims: nprob triples nx, ny, nz).  Every operator of the V-cycle and of the
  * CG runs as one launch per (operator, level, colour) across all problems,
  * with per-problem reductions, scalars and convergence; one batched CG
- * iteration is one hipGraph. */
+ * iteration is one hipGraph.  A solve takes at most 65535 problems. */
 typedef struct hpcgx_batch hpcgx_batch;
 int hpcgx_batch_create(int nprob, const int* dims, int nlevels, int stores, void* stream, hpcgx_batch** out);
 int hpcgx_batch_destroy(hpcgx_batch* b);

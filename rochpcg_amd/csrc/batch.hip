@@ -219,7 +219,7 @@ struct Planner
         return w;
     }
 
-    // append a launch whose segments are built by `fill(k, seg) -> bool`
+    // append the launch (launch_end: or launches) whose segments are built by `fill(k, seg) -> bool`
     template <typename Fill>
     int add(int kind, int block, bool vector_kind, int r_f64, int dot, double beta, Fill&& fill)
     {
@@ -235,12 +235,41 @@ struct Planner
                 segs.push_back(sg);
                 prob.push_back(k);
             }
-        const int rows = launch_rows(segs.data(), segs.size(), next_rows);
-        const int64_t nb = assign_blocks(segs.data(), segs.size(), block, vector_kind, rows);
+        BLaunch L;
+        std::memset(&L, 0, sizeof(L));
+        L.kind = kind;
+        L.prec = prec;
+        L.r_f64 = r_f64;
+        L.dot = dot;
+        L.block = block;
+        L.beta = beta;
+        L.bf32 = next_bf32;
+        L.win = next_win;
+        L.win_tail = next_tail;
+        L.all_u = next_all_u;
+        L.rows = launch_rows(segs.data(), segs.size(), next_rows);
+        next_subs = 1;
+        next_bf32 = 0;
+        next_win = next_tail = W;
+        next_all_u = 0;
+        next_rows = 1;
+        for(size_t j0 = 0, e; j0 < segs.size(); j0 = e)
+        {
+            e = launch_end(prob, j0);
+            HPCGX_TRY(add_launch(L, segs.data() + j0, prob.data() + j0, e - j0, vector_kind));
+        }
+        return 0;
+    }
+
+    // append launch L over nseg segments
+    int add_launch(BLaunch L, BSeg* segs, const size_t* prob, size_t nseg, bool vector_kind)
+    {
+        L.nseg = (int)nseg;
+        L.nblocks = assign_blocks(segs, nseg, L.block, vector_kind, L.rows);
+        L.pat = L.kind <= BK_RESTRICT;
         // the segments of a problem follow each other: their partials too, and
         // the first folds them all
-        int pat = kind <= BK_RESTRICT;
-        for(size_t j = 0, first = 0; j < segs.size(); ++j)
+        for(size_t j = 0, first = 0; j < nseg; ++j)
         {
             if(prob[j] != prob[first]) first = j;
             segs[j].part0 = segs[first].nfold;
@@ -250,51 +279,17 @@ struct Planner
                 set_error("batched reduction exceeds the partial capacity");
                 return -2;
             }
-            if(!segs[j].cols.pat) pat = 0;
+            if(!segs[j].cols.pat) L.pat = 0;
+            L.nrows += segs[j].size;
+            if(segs[j].t) L.any_t = 1;
         }
-        BLaunch L;
-        std::memset(&L, 0, sizeof(L));
-        for(const BSeg& sg : segs)
-        {
-            L.nrows += sg.size;
-            if(sg.t) L.any_t = 1;
-        }
-        L.kind = kind;
-        L.prec = prec;
-        L.r_f64 = r_f64;
-        L.dot = dot;
-        L.block = block;
-        L.nseg = (int)segs.size();
-        L.nblocks = nb;
-        L.beta = beta;
-        L.bf32 = next_bf32;
-        L.win = next_win;
-        L.win_tail = next_tail;
-        L.all_u = next_all_u;
-        L.rows = rows;
-        L.pat = pat;
-        next_subs = 1;
-        next_bf32 = 0;
-        next_win = next_tail = W;
-        next_all_u = 0;
-        next_rows = 1;
-        if(!segs.empty())
-        {
-            if(segs.size() > MAX_SEGS)
-            {
-                set_error("too many problems in one batched launch");
-                return -2;
-            }
-            std::vector<char> h(table_bytes(segs.size(), nb));
-            std::memcpy(h.data(), segs.data(), sizeof(BSeg) * segs.size());
-            block_map(segs.data(), segs.size(), reinterpret_cast<uint16_t*>(h.data() + sizeof(BSeg) * segs.size()));
-            BSeg* d = nullptr;
-            HPCGX_HIP(hipMalloc(&d, h.size() + 2));   // seg_of reads whole words of the map
-            B.tables.push_back(d);
-            HPCGX_HIP(hipMemcpy(d, h.data(), h.size(), hipMemcpyHostToDevice));
-            L.segs = d;
-            out->push_back(L);
-        }
+        std::vector<char> h(table_bytes(nseg, L.nblocks));
+        std::memcpy(h.data(), segs, sizeof(BSeg) * nseg);
+        block_map(segs, nseg, reinterpret_cast<uint16_t*>(h.data() + sizeof(BSeg) * nseg));
+        HPCGX_HIP(hipMalloc((void**)&L.segs, h.size() + 2));   // seg_of reads whole words of the map
+        B.tables.push_back(L.segs);
+        HPCGX_HIP(hipMemcpy(L.segs, h.data(), h.size(), hipMemcpyHostToDevice));
+        out->push_back(L);
         return 0;
     }
 
@@ -522,6 +517,11 @@ struct Planner
 
 static int plan(Batch& B)
 {
+    if(B.probs.size() > MAX_SEGS)   // a segment each in the vector launches
+    {
+        set_error("too many problems in one batch");
+        return -2;
+    }
     for(int mode = 0; mode < 2; ++mode)
     {
         const bool mixed = mode == CG_MIXED;

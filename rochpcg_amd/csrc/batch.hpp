@@ -41,10 +41,23 @@ struct BSeg
 // every logical block, one uint16 each (map[b] = j for b in [blk0_j, blk0_j +
 // nblk_j)), so a block finds its segment with one load instead of a search.
 constexpr size_t MAX_SEGS = 65535;
+static_assert(MAX_COLORS < MAX_SEGS, "a launch holds a problem's segments");
 
 __host__ __device__ inline const uint16_t* seg_map(const BSeg* segs, int nseg)
 {
     return reinterpret_cast<const uint16_t*>(segs + nseg);
+}
+
+// A launch takes as many whole problems as its block map can name segments of:
+// where the segments of all (prob[j] is segment j's problem) are more, as in the
+// SpMV's of one segment a colour from 8192 problems of eight colours on, several
+// launches follow each other.  The end of the one that starts at segment j0.
+inline size_t launch_end(const std::vector<size_t>& prob, size_t j0)
+{
+    size_t e = prob.size() - j0 > MAX_SEGS ? j0 + MAX_SEGS : prob.size();
+    if(e < prob.size())
+        while(prob[e] == prob[e - 1]) --e;   // a problem has MAX_COLORS segments at most
+    return e;
 }
 
 inline size_t table_bytes(size_t nseg, int64_t nblocks) { return sizeof(BSeg) * nseg + 2 * (size_t)nblocks; }
