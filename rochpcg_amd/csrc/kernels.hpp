@@ -155,13 +155,16 @@ __device__ __forceinline__ void block_reduce(double v, const RedArgs& ra)
 // Vector loads of R consecutive rows of one ELL slot.  A thread owns rows
 // [row, row+R) (row % R == 0, m % R == 0), so a wave issues one contiguous
 // 64*R-element segment per slot: dwordx2/x4 loads instead of R dword loads.
+// The vector types are aligned as their elements are: callers' vectors need no
+// more than that (gfx950 loads and stores dwordx2/x4 at any element's address, so
+// the instructions are the same).
 template <typename T, int R>
 struct Ext;
 #define HPCGX_EXT(T, R) \
     template <>         \
     struct Ext<T, R>    \
     {                   \
-        typedef T type __attribute__((ext_vector_type(R))); \
+        typedef T type __attribute__((ext_vector_type(R), aligned(sizeof(T)))); \
     };
 HPCGX_EXT(int32_t, 2)
 HPCGX_EXT(int32_t, 4)
@@ -172,6 +175,8 @@ HPCGX_EXT(float, 4)
 HPCGX_EXT(uint16_t, 2)
 HPCGX_EXT(uint16_t, 4)
 #undef HPCGX_EXT
+static_assert(alignof(Ext<double, 2>::type) == alignof(double) && alignof(Ext<float, 2>::type) == alignof(float),
+              "callers' vectors are aligned as their elements");
 
 template <int R, typename T>
 __device__ __forceinline__ void ld_nt(const T* p, T (&o)[R])
