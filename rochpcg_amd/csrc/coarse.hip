@@ -12,15 +12,18 @@
 // instruction every four cycles): so the columns are laid out beforehand as LDS
 // offsets, by section, with the unused slots of a group pointing at a zero
 // behind the level's x.  A sum is then one LDS read and one multiply-add a
-// slot, without masks or selects; the rest is a division and a barrier.
+// slot, without masks or selects; the rest is a division and a barrier.  A sum that
+// comes out as NaN is taken again with the unused slots left out (sum_used): the
+// value of an unused slot, which may be infinite, is no part of it.
 //
 // Measured, a CG iteration of FP64 / mixed with every level as launches and with
 // its coarse levels here: 16^3 254 / 238 -> 148 / 114 us, 32^3 282 / 254 ->
 // 220 / 171 us, 64^3 382 / 313 -> 358 / 268 us, 104^3 561 / 418 -> 545 / 391 us;
 // a step takes 0.5-0.9 us.
 //
-// Per row the arithmetic is that of the row_* functions of kernels.hpp, slot by
-// slot in the same order (an unused slot adds a * 0), so results are the same.
+// Per row the arithmetic is that of the row_* functions of kernels.hpp, on the same
+// stored values, slot by slot in the same order (an unused slot adds a * 0), so
+// results are the same (but for the sign of a sum that is zero).
 // The inner levels' r and x are left in the level vectors, as the launches leave
 // them.
 //
@@ -166,13 +169,30 @@ __device__ __forceinline__ void sum_groups(const char* xs, int j0, int n, const 
     }
 }
 
+// The same sum over the groups' used slots alone, straight from memory.
+template <typename VT, typename XT>
+__device__ __forceinline__ XT sum_used(ConstLevel& L, const char* xs, int gv, int gi, int n, int row, XT s)
+{
+    const uint32_t unused = (uint32_t)L.m * (uint32_t)sizeof(XT);
+#pragma unroll 1
+    for(int p = 0; p < 4 * n; ++p)
+    {
+        const uint32_t at = ((const uint16_t*)(L.at + (int64_t)(gi + p / 4) * L.m + row))[p % 4];
+        if(at != unused) s = fmaT(-cvt<XT>(((const VT*)L.val)[ell_at(4 * gv + p, row)]), *(const XT*)(xs + at), s);
+    }
+    return s;
+}
+
 template <typename VT, typename XT>
 __device__ __forceinline__ void coarse_load(ConstLevel& L, const void* r, bool r_f64, const CoarseStep& S, int row,
                                             CoarseRow<VT, XT>& o)
 {
     load_groups<0, VT, XT>(group_ptr<VT>(L, S.va, S.ia), group_ptr<VT>(L, S.vb, S.ib), S.na, S.na + S.nb, 8 * L.m,
                            (uint32_t)(ell_at(0, row) * sizeof(VT)), 8u * (uint32_t)row, o);
-    o.d = ((const VT*)L.dg)[row];
+    if(S.kind == CK_FWD_T)   // as row_fwd_full, which has the whole row at hand
+        o.d = ((const VT*)L.val)[ell_at(L.diag_idx[row], row)];
+    else
+        o.d = ((const VT*)L.dg)[row];
     if(S.kind == CK_FWD || S.kind >= CK_FWD_T)
     {
         if(r_f64)
@@ -183,7 +203,7 @@ __device__ __forceinline__ void coarse_load(ConstLevel& L, const void* r, bool r
 }
 
 template <typename VT, typename XT>
-__device__ __forceinline__ void coarse_compute(char* xs, XT* ts, bool r_f64, const CoarseStep& S, int row,
+__device__ __forceinline__ void coarse_compute(ConstLevel& L, char* xs, XT* ts, bool r_f64, const CoarseStep& S, int row,
                                                const CoarseRow<VT, XT>& o)
 {
 #pragma clang fp contract(off)
@@ -200,6 +220,16 @@ __device__ __forceinline__ void coarse_compute(char* xs, XT* ts, bool r_f64, con
         ts[row] = S.kind == CK_BWD_ZERO_U ? s0 - s : s;
         if(S.kind == CK_FWD_U) s = s - u;
         sum_groups<0, VT, XT>(xs, S.na, S.na + S.nb, o, s);
+    }
+    if(s != s)
+    {
+        s = sum_used<VT, XT>(L, xs, S.va, S.ia, S.na, row, s0);
+        if(S.kind >= CK_BWD_ZERO_U)
+        {
+            ts[row] = S.kind == CK_BWD_ZERO_U ? s0 - s : s;
+            if(S.kind == CK_FWD_U) s = s - u;
+            s = sum_used<VT, XT>(L, xs, S.vb, S.ib, S.nb, row, s);
+        }
     }
     *mine = s / d;
 }
@@ -238,7 +268,7 @@ __device__ __forceinline__ void coarse_symgs(ConstLevel& L, char* lds, const voi
         next = step_at(steps + min(k + T, n - 1));
 #pragma unroll 1
         for(; passed < k; ++passed) __syncthreads();
-        if(any && lane < S.n) coarse_compute<VT, XT>(xs, ts, r_f64, S, S.off + lane, o);
+        if(any && lane < S.n) coarse_compute<VT, XT>(L, xs, ts, r_f64, S, S.off + lane, o);
         __syncthreads();
         ++passed;
     }
@@ -256,16 +286,13 @@ __device__ __forceinline__ void coarse_restrict(ConstLevel& L, ConstLevel& C, ch
     {
         const int row = L.f2c_fine[k];
         CoarseRow<VT, XT> o;
-        const GroupPtr g = group_ptr<VT>(L, 0, SEC_LOWER * GROUPS);
+        const GroupPtr g = group_ptr<VT>(L, 0, SEC_ROW * GROUPS);
         load_groups<0, VT, XT>(g, g, GROUPS, GROUPS, 8 * m, (uint32_t)(ell_at(0, row) * sizeof(VT)), 8u * (uint32_t)row,
                                o);
-        const VT d = ((const VT*)L.dg)[row];
-        XT s = r_f64 ? (XT)((const double*)r)[row] : ((const XT*)r)[row];
+        const XT s0 = r_f64 ? (XT)((const double*)r)[row] : ((const XT*)r)[row];
+        XT s = s0;
         sum_groups<0, VT, XT>(xs, 0, GROUPS, o, s);
-        s = fmaT(-cvt<XT>(d), ((const XT*)xs)[row], s);
-#pragma unroll
-        for(int g = 0; g < GROUPS; ++g) o.at[g] = L.at[(SEC_UPPER * GROUPS + g) * m + row];
-        sum_groups<0, VT, XT>(xs, 0, GROUPS, o, s);
+        if(s != s) s = sum_used<VT, XT>(L, xs, 0, SEC_ROW * GROUPS, GROUPS, row, s0);
         ((XT*)C.r)[L.f2c_coarse[k]] = s;
     }
     __syncthreads();
@@ -339,7 +366,7 @@ __global__ __launch_bounds__(256) void k_coarse_columns(int m, int xbytes, const
     {
         const int c = p < W ? col[ell_at(p, row)] : -1;
         const bool up = p < W && p >= desc_upper(ds), tail = p < W && p >= desc_tail(ds);
-        const bool in[SEC_COUNT] = {p < desc_diag(ds), up, up && !tail, tail};
+        const bool in[SEC_COUNT] = {p < desc_diag(ds), up, up && !tail, tail, p <= desc_diag(ds) || up};
         for(int s = 0; s < SEC_COUNT; ++s)
             at[(((int64_t)s * GROUPS + p / 4) * m + row) * 4 + p % 4] = (uint16_t)((in[s] ? c : m) * xbytes);
     }
@@ -446,6 +473,7 @@ static int build_plan(Problem& P, Prec prec)
         const LevelVecs& V = prec == PREC_F64 ? P.v64[l] : P.v32[l];
         h[j].val = prec == PREC_F64 ? (const void*)L.ell_val : (const void*)L.ell_h;
         h[j].dg = prec == PREC_F64 ? (const void*)L.diag64 : (const void*)L.diag_h;
+        h[j].diag_idx = L.diag_idx;
         h[j].at = (const uint2*)((uint16_t*)mem + cols[j]);
         h[j].f2c_fine = L.f2c_fine;
         h[j].f2c_coarse = L.f2c_coarse;

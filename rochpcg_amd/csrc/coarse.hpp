@@ -5,15 +5,16 @@
 namespace hpcgx
 {
 
-// Sections of a row's entries: left of the diagonal, right of it, and of these
-// the ones outside and inside the last colour.
+// Sections of a row's entries: left of the diagonal, right of it, of these the
+// ones outside and inside the last colour, and the row as a whole.
 enum CoarseSection : int
 {
     SEC_LOWER = 0,
     SEC_UPPER = 1,
     SEC_MID = 2,
     SEC_TAIL = 3,
-    SEC_COUNT = 4
+    SEC_ROW = 4,
+    SEC_COUNT = 5
 };
 
 // One step of a symmetric Gauss-Seidel sweep over a level: some rows of one
@@ -32,6 +33,7 @@ struct CoarseLevel
 {
     const void* val;           // values, and diagonal
     const void* dg;
+    const int32_t* diag_idx;   // slot of the diagonal
     const uint2* at;           // LDS byte offsets of the columns' x, 16 bits each: [section][group][row]
     const int32_t* f2c_fine;   // to the next level
     const int32_t* f2c_coarse;
