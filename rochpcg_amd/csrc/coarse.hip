@@ -12,9 +12,9 @@
 // instruction every four cycles): so the columns are laid out beforehand as LDS
 // offsets, by section, with the unused slots of a group pointing at a zero
 // behind the level's x.  A sum is then one LDS read and one multiply-add a
-// slot, without masks or selects; the rest is a division and a barrier.  A sum that
-// comes out as NaN is taken again with the unused slots left out (sum_used): the
-// value of an unused slot, which may be infinite, is no part of it.
+// slot, without masks or selects; the rest is a division and a barrier.  The value
+// of an unused slot may be infinite, though it is no part of the sum: where any sum
+// has come out as NaN, the V-cycle is run again over the used slots alone (CM_USED).
 //
 // Measured, a CG iteration of FP64 / mixed with every level as launches and with
 // its coarse levels here: 16^3 254 / 238 -> 148 / 114 us, 32^3 282 / 254 ->
@@ -39,7 +39,8 @@ namespace hpcgx
 
 constexpr int COARSE_TEAMS = 4;               // see coarse_symgs
 // threads of a team, the most rows of a step: as many as leave a row's operands
-// in registers
+// in registers (FP64 takes 153 of the 168 that 12 waves may have, mixed 94 of 128;
+// no scratch)
 template <typename XT>
 constexpr int coarse_team() { return sizeof(XT) == 8 ? 192 : 256; }
 template <typename XT>
@@ -169,7 +170,15 @@ __device__ __forceinline__ void sum_groups(const char* xs, int j0, int n, const 
     }
 }
 
-// The same sum over the groups' used slots alone, straight from memory.
+// How a level's steps are run
+enum CoarseMode : int
+{
+    CM_PLAIN,   // no CK_FWD_T among them
+    CM_ROWS,    // CK_FWD_T takes the diagonal of the row, as row_fwd_full does
+    CM_USED     // every sum over its used slots alone
+};
+
+// The sum over the groups' used slots, straight from memory.
 template <typename VT, typename XT>
 __device__ __forceinline__ XT sum_used(ConstLevel& L, const char* xs, int gv, int gi, int n, int row, XT s)
 {
@@ -183,13 +192,14 @@ __device__ __forceinline__ XT sum_used(ConstLevel& L, const char* xs, int gv, in
     return s;
 }
 
-template <typename VT, typename XT>
+template <int MODE, typename VT, typename XT>
 __device__ __forceinline__ void coarse_load(ConstLevel& L, const void* r, bool r_f64, const CoarseStep& S, int row,
                                             CoarseRow<VT, XT>& o)
 {
-    load_groups<0, VT, XT>(group_ptr<VT>(L, S.va, S.ia), group_ptr<VT>(L, S.vb, S.ib), S.na, S.na + S.nb, 8 * L.m,
-                           (uint32_t)(ell_at(0, row) * sizeof(VT)), 8u * (uint32_t)row, o);
-    if(S.kind == CK_FWD_T)   // as row_fwd_full, which has the whole row at hand
+    if constexpr(MODE != CM_USED)
+        load_groups<0, VT, XT>(group_ptr<VT>(L, S.va, S.ia), group_ptr<VT>(L, S.vb, S.ib), S.na, S.na + S.nb, 8 * L.m,
+                               (uint32_t)(ell_at(0, row) * sizeof(VT)), 8u * (uint32_t)row, o);
+    if(MODE != CM_PLAIN && S.kind == CK_FWD_T)
         o.d = ((const VT*)L.val)[ell_at(L.diag_idx[row], row)];
     else
         o.d = ((const VT*)L.dg)[row];
@@ -202,9 +212,10 @@ __device__ __forceinline__ void coarse_load(ConstLevel& L, const void* r, bool r
     }
 }
 
-template <typename VT, typename XT>
+// nan becomes NaN with a sum that is one
+template <int MODE, typename VT, typename XT>
 __device__ __forceinline__ void coarse_compute(ConstLevel& L, char* xs, XT* ts, bool r_f64, const CoarseStep& S, int row,
-                                               const CoarseRow<VT, XT>& o)
+                                               const CoarseRow<VT, XT>& o, XT& nan)
 {
 #pragma clang fp contract(off)
     XT* mine = (XT*)xs + row;
@@ -214,23 +225,21 @@ __device__ __forceinline__ void coarse_compute(ConstLevel& L, char* xs, XT* ts, 
     if(S.kind == CK_BWD_ZERO || S.kind == CK_BWD_ZERO_U) s = *mine * d;
     if(S.kind == CK_FWD_U) u = ts[row];
     const XT s0 = s;
-    sum_groups<0, VT, XT>(xs, 0, S.na, o, s);
+    if constexpr(MODE == CM_USED)
+        s = sum_used<VT, XT>(L, xs, S.va, S.ia, S.na, row, s);
+    else
+        sum_groups<0, VT, XT>(xs, 0, S.na, o, s);
     if(S.kind >= CK_BWD_ZERO_U)
     {
         ts[row] = S.kind == CK_BWD_ZERO_U ? s0 - s : s;
         if(S.kind == CK_FWD_U) s = s - u;
-        sum_groups<0, VT, XT>(xs, S.na, S.na + S.nb, o, s);
-    }
-    if(s != s)
-    {
-        s = sum_used<VT, XT>(L, xs, S.va, S.ia, S.na, row, s0);
-        if(S.kind >= CK_BWD_ZERO_U)
-        {
-            ts[row] = S.kind == CK_BWD_ZERO_U ? s0 - s : s;
-            if(S.kind == CK_FWD_U) s = s - u;
+        if constexpr(MODE == CM_USED)
             s = sum_used<VT, XT>(L, xs, S.vb, S.ib, S.nb, row, s);
-        }
+        else
+            sum_groups<0, VT, XT>(xs, S.na, S.na + S.nb, o, s);
     }
+    // a multiply-add a row; a look at each sum on the spot made 64^3 mixed 1.5% slower
+    nan = fmaT((XT)0, s, nan);
     *mine = s / d;
 }
 
@@ -243,8 +252,8 @@ __device__ __forceinline__ CoarseStep step_at(ConstStep* s)
 // take them in turn; a barrier ends every step.  A team issues the loads of its
 // next step right after it has computed one, T - 1 barriers ahead of their use.
 // Every wave passes n = k1 - k0 barriers.
-template <typename VT, typename XT>
-__device__ __forceinline__ void coarse_symgs(ConstLevel& L, char* lds, const void* r, bool r_f64, int k0, int k1)
+template <int MODE, typename VT, typename XT>
+__device__ __forceinline__ void coarse_symgs(ConstLevel& L, char* lds, const void* r, bool r_f64, int k0, int k1, XT& nan)
 {
     constexpr int T = COARSE_TEAMS;
     const int team = __builtin_amdgcn_readfirstlane((int)threadIdx.x / coarse_team<XT>());
@@ -264,11 +273,11 @@ __device__ __forceinline__ void coarse_symgs(ConstLevel& L, char* lds, const voi
         // threads past the step's rows load its last row and store nothing; waves
         // past them do neither
         const bool any = wave < S.n;
-        if(any) coarse_load<VT, XT>(L, r, r_f64, S, S.off + min(lane, S.n - 1), o);
+        if(any) coarse_load<MODE, VT, XT>(L, r, r_f64, S, S.off + min(lane, S.n - 1), o);
         next = step_at(steps + min(k + T, n - 1));
 #pragma unroll 1
         for(; passed < k; ++passed) __syncthreads();
-        if(any && lane < S.n) coarse_compute<VT, XT>(L, xs, ts, r_f64, S, S.off + lane, o);
+        if(any && lane < S.n) coarse_compute<MODE, VT, XT>(L, xs, ts, r_f64, S, S.off + lane, o, nan);
         __syncthreads();
         ++passed;
     }
@@ -278,21 +287,26 @@ __device__ __forceinline__ void coarse_symgs(ConstLevel& L, char* lds, const voi
 
 // rc = the residual at the injected rows (row_restrict), into the next level's r
 template <typename VT, typename XT>
-__device__ __forceinline__ void coarse_restrict(ConstLevel& L, ConstLevel& C, char* lds, const void* r, bool r_f64)
+__device__ __forceinline__ void coarse_restrict(ConstLevel& L, ConstLevel& C, char* lds, const void* r, bool r_f64,
+                                                bool used, XT& nan)
 {
     const int mc = L.mc, m = L.m;
     const char* xs = lds + L.lds_x;
     for(int k = threadIdx.x; k < mc; k += coarse_bs<XT>())
     {
         const int row = L.f2c_fine[k];
-        CoarseRow<VT, XT> o;
-        const GroupPtr g = group_ptr<VT>(L, 0, SEC_ROW * GROUPS);
-        load_groups<0, VT, XT>(g, g, GROUPS, GROUPS, 8 * m, (uint32_t)(ell_at(0, row) * sizeof(VT)), 8u * (uint32_t)row,
-                               o);
-        const XT s0 = r_f64 ? (XT)((const double*)r)[row] : ((const XT*)r)[row];
-        XT s = s0;
-        sum_groups<0, VT, XT>(xs, 0, GROUPS, o, s);
-        if(s != s) s = sum_used<VT, XT>(L, xs, 0, SEC_ROW * GROUPS, GROUPS, row, s0);
+        XT s = r_f64 ? (XT)((const double*)r)[row] : ((const XT*)r)[row];
+        if(used)
+            s = sum_used<VT, XT>(L, xs, 0, SEC_ROW * GROUPS, GROUPS, row, s);
+        else
+        {
+            CoarseRow<VT, XT> o;
+            const GroupPtr g = group_ptr<VT>(L, 0, SEC_ROW * GROUPS);
+            load_groups<0, VT, XT>(g, g, GROUPS, GROUPS, 8 * m, (uint32_t)(ell_at(0, row) * sizeof(VT)),
+                                   8u * (uint32_t)row, o);
+            sum_groups<0, VT, XT>(xs, 0, GROUPS, o, s);
+        }
+        nan = fmaT((XT)0, s, nan);
         ((XT*)C.r)[L.f2c_coarse[k]] = s;
     }
     __syncthreads();
@@ -305,6 +319,8 @@ __device__ __forceinline__ void coarse_vcycle(const CoarseRun& R, char* lds)
     // the zero that unused slots read
     for(int l = threadIdx.x; l < R.nl; l += coarse_bs<XT>()) ((XT*)(lds + R.lv[l].lds_x))[R.lv[l].m] = 0;
     __syncthreads();
+    XT nan = 0;
+    bool used = false;
     // down, then up again; the bottom is its own way up
 #pragma unroll 1
     for(int v = 0; v < 2 * R.nl - 1; ++v)
@@ -315,7 +331,7 @@ __device__ __forceinline__ void coarse_vcycle(const CoarseRun& R, char* lds)
         ConstLevel& L = lv[l];
         XT* xs = (XT*)(lds + L.lds_x);
         const void* r = l == 0 ? R.r : L.r;
-        const bool r64 = l == 0 && R.r_f64;
+        const bool r64 = sizeof(XT) < sizeof(double) && l == 0 && R.r_f64;
         if(up)
         {
             const XT* xc = (const XT*)(lds + lv[l + 1].lds_x);
@@ -327,10 +343,23 @@ __device__ __forceinline__ void coarse_vcycle(const CoarseRun& R, char* lds)
             }
             __syncthreads();
         }
-        coarse_symgs<VT, XT>(L, lds, r, r64, up ? L.npre : 0, up ? L.npre + L.npost : L.npre);
-        if(!up && !bottom) coarse_restrict<VT, XT>(L, lv[l + 1], lds, r, r64);
+        const int k0 = up ? L.npre : 0, k1 = up ? L.npre + L.npost : L.npre;
+        if(used)
+            coarse_symgs<CM_USED, VT, XT>(L, lds, r, r64, k0, k1, nan);
+        else if(up && L.whole_rows)
+            coarse_symgs<CM_ROWS, VT, XT>(L, lds, r, r64, k0, k1, nan);
+        else
+            coarse_symgs<CM_PLAIN, VT, XT>(L, lds, r, r64, k0, k1, nan);
+        if(!up && !bottom) coarse_restrict<VT, XT>(L, lv[l + 1], lds, r, r64, used, nan);
         if(up || bottom)
         {
+            // before the result is written: r may be x
+            if(l == 0 && !used && __syncthreads_or(nan != nan))
+            {
+                used = true;
+                v = -1;
+                continue;
+            }
             XT* x = (XT*)(l == 0 ? R.x : L.x);
             const int m = L.m;
             for(int i = threadIdx.x; i < m; i += coarse_bs<XT>()) x[i] = xs[i];
@@ -481,6 +510,7 @@ static int build_plan(Problem& P, Prec prec)
         h[j].r = V.r;
         h[j].x = V.x;
         h[j].m = (int)L.m;
+        h[j].whole_rows = !L.u_ok;
         h[j].mc = j + 1 < nc ? (int)L.mc : 0;
         hipLaunchKernelGGL(k_coarse_columns, dim3((unsigned)ceil_div(L.m, 256)), dim3(256), 0, P.s, (int)L.m,
                            prec == PREC_F64 ? 8 : 4, L.ell_col, L.desc, (uint16_t*)mem + cols[j]);

@@ -41,6 +41,7 @@ struct CoarseLevel
     void* r;                   // the level's vectors (level 0: given with the launch)
     void* x;
     int m, mc, npre, npost;
+    int whole_rows;            // the post-smoother has steps of kind CK_FWD_T
     int lds_x, lds_t;          // where the level's x and t lie in LDS (bytes)
 };
 

@@ -69,3 +69,41 @@ def test_diagonals_of_the_rows(hip, dims, nlevels):
             V[ell].upload(a)
     _same_either_way(hip, G)
     G.close()
+
+
+@pytest.mark.parametrize("dims,nlevels", [((32, 32, 32), 4), ((20, 12, 8), 1)])
+def test_special_values_in_the_rhs(hip, dims, nlevels):
+    """Infinities and NaN in r reach the rows that the launches let them reach; a
+    one-level V-cycle may overwrite its rhs, also when it is run again."""
+    G = hip.Problem(*dims, nlevels=nlevels, stores=hip.STORE_F64 | hip.STORE_MIXED)
+    r = np.random.default_rng(5).uniform(-1, 1, G.m)
+    special = r.copy()
+    special[[3, G.m // 2, G.m - 2]] = [np.inf, np.nan, -np.inf]
+    last = G.color_table(nlevels - 1)[1][G.levels[nlevels - 1].ncolors - 1]
+    slots, V = _diagonal_slots(G, nlevels - 1), G.level_views(nlevels - 1)
+
+    def results():
+        out = []
+        for rhs in (r, special):
+            dr, y, z = hip.DeviceArray.from_host(rhs), hip.DeviceArray(G.m), hip.DeviceArray(G.m, np.float32)
+            G.mg(dr, y)
+            G.mg_mixed(dr, z)
+            out += [y.host(), z.host()]
+            if nlevels == 1:
+                G.mg(dr, dr)
+                out.append(dr.host())
+        return out
+
+    for infinite in (False, True):
+        if infinite:
+            a, d = V["ell_val"].host(), V["diag"].host()
+            a[slots[last:]] = np.inf
+            d[last:] = np.inf
+            V["ell_val"].upload(a)
+            V["diag"].upload(d)
+        G.set_coarse_rows(0)
+        want = results()
+        G.set_coarse_rows(8191)
+        for k, (a, b) in enumerate(zip(results(), want)):
+            assert np.array_equal(a, b, equal_nan=True), (infinite, k)
+    G.close()
