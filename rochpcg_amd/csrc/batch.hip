@@ -566,6 +566,8 @@ static int plan(Batch& B)
         }));
     }
     B.planned = true;
+    B.routes.clear();
+    for(const Problem* P : B.probs) B.routes.push_back(P->routes);
     return 0;
 }
 
@@ -585,6 +587,19 @@ static void free_plans(Batch& B)
     for(void* t : B.tables) (void)hipFree(t);
     B.tables.clear();
     B.planned = false;
+}
+
+// the plans as the problems' switches are now
+static int ensure_plan(Batch& B)
+{
+    bool same = B.planned;
+    for(size_t k = 0; same && k < B.probs.size(); ++k) same = B.probs[k]->routes == B.routes[k];
+    if(same) return 0;
+    HPCGX_HIP(hipStreamSynchronize(B.s));
+    free_plans(B);
+    const int rc = plan(B);
+    if(rc) free_plans(B);
+    return rc;
 }
 
 int batch_create(Batch*& out, int nprob, const int* dims, int nlevels, bool with_f64, bool with_mixed, hipStream_t s)
@@ -743,7 +758,7 @@ int batch_profile(Batch& B, int mode, int iters, double* kind_ms, double* kind_b
         set_error("invalid CG mode");
         return -2;
     }
-    if(!B.planned) HPCGX_TRY(plan(B));
+    HPCGX_TRY(ensure_plan(B));
     const std::vector<BLaunch>& it = B.iter[mode];
     if(it.empty())
     {
@@ -818,7 +833,7 @@ int batch_cg(Batch& B, int mode, int max_iter, double tol, bool use_graph, int* 
         set_error("invalid CG mode");
         return -2;
     }
-    if(!B.planned) HPCGX_TRY(plan(B));
+    HPCGX_TRY(ensure_plan(B));
     if(B.iter[mode].empty())
     {
         set_error("the batch was built without the store this mode needs");

@@ -159,6 +159,7 @@ struct Batch
     std::vector<void*> tables;              // device allocations of the plans
     std::vector<BLaunch> pre[2], iter[2];   // preamble and one iteration, per CG mode
     bool planned = false;
+    std::vector<unsigned> routes;           // the problems' Problem::routes at planning
     hipGraph_t graph[2] = {nullptr, nullptr};
     hipGraphExec_t gexec[2] = {nullptr, nullptr};
     int host_iter = 0;

@@ -609,6 +609,7 @@ int hpcgx_set_row_patterns(hpcgx_problem* p, int level, int on)
     }
     for(int l = 0; l < p->P->nlevels; ++l)
         if(level < 0 || l == level) p->P->L[l].pat_off = on == 0;
+    ++p->P->routes;
     p->P->invalidate_graphs();
     return 0;
 }
@@ -622,6 +623,7 @@ int hpcgx_set_coarse_rows(hpcgx_problem* p, int rows)
         return -2;
     }
     p->P->coarse_rows = rows;
+    ++p->P->routes;
     p->P->invalidate_graphs();
     return 0;
 }

@@ -91,6 +91,7 @@ struct Problem
     int graph_replace = -1;
     CoarsePlan coarse[2];     // [precision]
     int coarse_rows = -1;     // levels of at most this many rows run in one workgroup (-1: COARSE_ROWS)
+    unsigned routes = 0;      // changes of what the kernels run on (Level::pat_off, coarse_rows), which plans hold
     RefPath* ref = nullptr;   // natural-order work vectors of the reference path (refpath.hip)
 
     // forget captured graphs (launch shapes or operands changed)
