@@ -37,6 +37,12 @@ int HPCGX_ReferenceCG(const SparseMatrix& A, int max_iter, double tolerance, int
 long long HPCGX_CheckProblem(const SparseMatrix& A, const Vector* b, const Vector* x, const Vector* xexact,
                              long long* counts);
 
+// Has A's level read its columns where they lie (A.ell_col_ind) from here on.  The
+// kernels otherwise read them from copies that OptimizeProblem makes, which is
+// faster: a program that writes other columns there calls this once, before or
+// after.  Values and diagonals are read in place in any case.
+int HPCGX_ReadColumnsInPlace(const SparseMatrix& A);
+
 // TestCG's exaggeration of the diagonal and of b (TestCG.cpp:67-95): the entry
 // at position i is scaled by (g+2)*1e6 when its global row id g < 9 and by 1e6
 // otherwise.  Like the reference, g is the natural row id of position i

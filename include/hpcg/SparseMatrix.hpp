@@ -62,7 +62,9 @@ struct SparseMatrix_STRUCT
     // ELL storage, multicolour row order, sliced: rows in slices of 128, slice
     // s holding slot p of its rows at [(s*ell_width + p)*128, +128), so entry p
     // of row r sits at ((r/128)*ell_width + p)*128 + r%128 (64-bit offsets;
-    // the reference's ELL is column-major, p*localNumberOfRows + r)
+    // the reference's ELL is column-major, p*localNumberOfRows + r).  Columns
+    // written through ell_col_ind are followed after HPCGX_ReadColumnsInPlace
+    // (Extensions.hpp), values always
     local_int_t ell_width;
     local_int_t* ell_col_ind;
     double* ell_val;

@@ -84,10 +84,17 @@ int hpcgx_color_table(const hpcgx_problem* p, int level, int* sizes, int* offset
  * in bits 0-7, first slot of an off-diagonal last-colour column in bits 8-15,
  * first upper slot in bits 16-23, 27 when absent; no reference counterpart), diagonal
  * values f64 (or NULL) and f16 (or NULL) (no reference counterpart).  The
- * kernels read the columns from copies made with the problem (row patterns,
- * and the coarse levels' own), so columns and descriptors written through these
- * pointers are not followed; values and diagonals are read where they lie */
+ * kernels read the level's arrays where they lie from this call on, so what is
+ * written through the pointers is followed.  Columns and descriptors are
+ * otherwise read from copies made with the problem (row patterns, and the
+ * coarse levels' own), which is faster: a program that only reads, the
+ * permutation for instance, takes hpcgx_level_arrays_const;
+ * hpcgx_set_row_patterns(p, level, 1) says that columns and descriptors are as
+ * they were created, and has the copies read again */
 int hpcgx_level_arrays(const hpcgx_problem* p, int level, void** ptrs);
+/* the same pointers for reading, or for writing values and diagonals, which are
+ * read where they lie in any case */
+int hpcgx_level_arrays_const(const hpcgx_problem* p, int level, const void** ptrs);
 /* device pointers of the CG data and system: ptrs[0..7] = b, x, xexact, r,
  * z (f64, or NULL), p, Ap, z (f32 mixed-mode, or NULL)  (CGData.hpp:55-61) */
 int hpcgx_vectors(const hpcgx_problem* p, void** ptrs);
@@ -308,15 +315,17 @@ int hpcgx_set_sweep_columns(hpcgx_problem* p, int level, int columns);
  * from the column array -- where the level has them; 0 = from the column
  * array.  Results do not depend on it.  A level has row patterns when each of
  * its colours repeats at most 32 lists, as the parity colourings of even grids
- * do; other levels always read the column array.  level -1 applies to all. */
+ * do; other levels always read the column array, and so do those whose arrays
+ * hpcgx_level_arrays has handed out, until on is set again.  level -1 applies
+ * to all. */
 int hpcgx_set_row_patterns(hpcgx_problem* p, int level, int on);
 /* The V-cycle runs the levels of at most `rows` rows, together with all below
  * them, as one launch of one workgroup (no reference counterpart; a tuning
  * knob).  -1 = the default (5000 rows for the f64 store, 8191 for the mixed
  * one), 0 = every level as launches per colour.  A level whose x and row sums
  * do not fit a CU's LDS, or of a colouring with too many entries on both sides
- * of the diagonal, is run as launches whatever `rows` says.  Results do not
- * depend on it. */
+ * of the diagonal, or whose arrays hpcgx_level_arrays has handed out, is run as
+ * launches whatever `rows` says.  Results do not depend on it. */
 int hpcgx_set_coarse_rows(hpcgx_problem* p, int rows);
 int hpcgx_synchronize(hpcgx_problem* p);
 int hpcgx_malloc(void** ptr, size_t bytes);

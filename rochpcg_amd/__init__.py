@@ -53,6 +53,7 @@ def _load():
         "hpcgx_level_info": ([vp, i32, P(i64)], i32),
         "hpcgx_color_table": ([vp, i32, vp, vp, vp], i32),
         "hpcgx_level_arrays": ([vp, i32, P(vp)], i32),
+        "hpcgx_level_arrays_const": ([vp, i32, P(vp)], i32),
         "hpcgx_vectors": ([vp, P(vp)], i32),
         "hpcgx_make_rhs": ([vp, i32, C.c_uint64], i32),
         "hpcgx_check_problem": ([vp, i32, i32, P(i64)], i32),
@@ -193,6 +194,28 @@ class DeviceArray:
             pass
 
 
+class _ColumnView(DeviceArray):
+    """A level's columns or descriptors.  Whoever takes the address may write
+    there: from then on the kernels read them where they lie."""
+
+    def __init__(self, problem, level, n, dtype, ptr):
+        self._problem, self._level, self._ptr = problem, level, int(ptr)
+        super().__init__(n, dtype, ptr=ptr, owner=False)
+
+    @property
+    def ptr(self):
+        if self._ptr:
+            _check(lib.hpcgx_level_arrays(self._problem.h, self._level, (C.c_void_p * 13)()))
+        return self._ptr
+
+    @ptr.setter
+    def ptr(self, value):
+        self._ptr = value
+
+    def host(self, start=0, count=None):
+        return DeviceArray(self.n, self.dtype, ptr=self._ptr, owner=False).host(start, count)
+
+
 def ell_padded_rows(m):
     """Rows the sliced ELL arrays of an m-row level hold (m rounded up to a
     whole slice)."""
@@ -291,7 +314,7 @@ class Problem:
         arrays as (rows, 27), row by row."""
         L = self.levels[level]
         ptrs = (C.c_void_p * 13)()
-        _check(lib.hpcgx_level_arrays(self.h, level, ptrs))
+        _check(lib.hpcgx_level_arrays_const(self.h, level, ptrs))
         m, mc = L.m, L.mc
         me = ell_padded_rows(m)
 
@@ -315,10 +338,12 @@ class Problem:
 
     def level_views(self, level=0):
         """Device arrays of a level as non-owning DeviceArray views (no copy);
-        the ELL arrays are sliced (read rows with ell_rows)."""
+        the ELL arrays are sliced (read rows with ell_rows).  Columns and
+        descriptors that are written through their views are followed
+        (hpcgx_level_arrays, at the first use of a view's address)."""
         L = self.levels[level]
         ptrs = (C.c_void_p * 13)()
-        _check(lib.hpcgx_level_arrays(self.h, level, ptrs))
+        _check(lib.hpcgx_level_arrays_const(self.h, level, ptrs))
         m, mc = L.m, L.mc
         me = ell_padded_rows(m)
         spec = (("ell_col", 27 * me, np.int32), ("ell_val", 27 * me, np.float64),
@@ -326,7 +351,8 @@ class Problem:
                 ("perm", m, np.int32), ("colors", m, np.int32), ("f2c", mc, np.int32),
                 ("f2c_fine", mc, np.int32), ("f2c_coarse", mc, np.int32), ("desc", m, np.int32),
                 ("diag", m, np.float64), ("diag_f16", m, np.float16))
-        return {name: DeviceArray(n, dt, ptr=ptr, owner=False)
+        return {name: _ColumnView(self, level, n, dt, ptr) if name in ("ell_col", "desc")
+                else DeviceArray(n, dt, ptr=ptr, owner=False)
                 for (name, n, dt), ptr in zip(spec, ptrs) if ptr and n}
 
     def make_rhs(self, kind=0, seed=0):

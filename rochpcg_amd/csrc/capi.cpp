@@ -140,15 +140,29 @@ int hpcgx_color_table(const hpcgx_problem* p, int level, int* sizes, int* offset
     return 0;
 }
 
+static void level_pointers(const Level& L, const void** ptrs)
+{
+    const void* v[] = {L.ell_col, L.ell_val, L.ell_h, L.diag_idx, L.inv_diag, L.perm, L.colors, L.f2c_nat, L.f2c_fine,
+                       L.f2c_coarse, L.desc, L.diag64, L.diag_h};
+    for(int i = 0; i < 13; ++i) ptrs[i] = v[i];
+}
+
 int hpcgx_level_arrays(const hpcgx_problem* p, int level, void** ptrs)
 {
     CHECK_P(p);
     CHECK_LEVEL(p, level);
     CHECK_PTRS(ptrs);
-    const Level& L = p->P->L[level];
-    void* v[] = {L.ell_col, L.ell_val, L.ell_h, L.diag_idx, L.inv_diag, L.perm, L.colors, L.f2c_nat, L.f2c_fine,
-                 L.f2c_coarse, L.desc, L.diag64, L.diag_h};
-    for(int i = 0; i < 13; ++i) ptrs[i] = v[i];
+    level_pointers(p->P->L[level], const_cast<const void**>(ptrs));
+    expose_columns(*p->P, level);
+    return 0;
+}
+
+int hpcgx_level_arrays_const(const hpcgx_problem* p, int level, const void** ptrs)
+{
+    CHECK_P(p);
+    CHECK_LEVEL(p, level);
+    CHECK_PTRS(ptrs);
+    level_pointers(p->P->L[level], ptrs);
     return 0;
 }
 
@@ -608,7 +622,11 @@ int hpcgx_set_row_patterns(hpcgx_problem* p, int level, int on)
         return -2;
     }
     for(int l = 0; l < p->P->nlevels; ++l)
-        if(level < 0 || l == level) p->P->L[l].pat_off = on == 0;
+        if(level < 0 || l == level)
+        {
+            p->P->L[l].pat_off = on == 0;
+            if(on) p->P->L[l].exposed = false;
+        }
     ++p->P->routes;
     p->P->invalidate_graphs();
     return 0;

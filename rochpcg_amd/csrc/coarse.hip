@@ -545,7 +545,7 @@ int coarse_first(const Problem& P, Prec prec)
 {
     const int rows = P.coarse_rows < 0 ? COARSE_ROWS[prec] : P.coarse_rows;
     int l = P.nlevels;
-    while(l > 0 && l - 1 >= P.coarse[prec].first && P.L[l - 1].m <= rows) --l;
+    while(l > 0 && l - 1 >= P.coarse[prec].first && P.L[l - 1].m <= rows && !P.L[l - 1].exposed) --l;
     return l;
 }
 

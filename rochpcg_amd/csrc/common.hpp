@@ -152,6 +152,10 @@ struct Level
     int32_t* pat_tab = nullptr;   // [ncolors][PAT_MAX][PAT_QUADS*4], in the allocation of pat
     int npat = 0;                 // patterns of the colour that has most
     bool pat_off = false;         // the kernels read the column array all the same
+    // a caller may write the columns and descriptors (hpcgx_level_arrays,
+    // HPCGX_ReadColumnsInPlace): they are read where they lie, not from the copies
+    // made at setup (row patterns, the coarse levels' offsets)
+    bool exposed = false;
     double* inv_diag = nullptr;   // [m] 1/a_ii (f64)
     double* diag64 = nullptr;     // [m] a_ii (f64 levels)
     __half* diag_h = nullptr;     // [m] a_ii (mixed levels)
@@ -175,7 +179,7 @@ struct Level
 
     Shape shp[2][SH_COUNT];   // [precision][operator]
 
-    bool use_pat() const { return pat != nullptr && !pat_off; }
+    bool use_pat() const { return pat != nullptr && !pat_off && !exposed; }
     ColArgs cols(int c) const
     {
         return ColArgs{ell_col, desc, pat, pat_tab ? pat_tab + (int64_t)c * PAT_MAX * PAT_QUADS * 4 : nullptr, npat};

@@ -719,6 +719,15 @@ void CheckProblem(SparseMatrix& A, Vector* b, Vector* x, Vector* xexact)
                 c[CHECK_NNZ], c[CHECK_ROWS]);
 }
 
+int HPCGX_ReadColumnsInPlace(const SparseMatrix& A)
+{
+    Problem* P;
+    int l;
+    if(!level_of(A, P, l)) return 1;
+    expose_columns(*P, l);
+    return 0;
+}
+
 int HPCGX_TestCGScale(const SparseMatrix& A, Vector& diagonal, Vector& b)
 {
     Problem* P;

@@ -315,11 +315,10 @@ static bool replace_at(const Problem& P, int iter_index)
 
 static int ensure_graph(Problem& P, int g)
 {
-    const bool stale = P.gexec[g] == nullptr || P.graph_mode != P.mode || P.graph_precond != P.precond ||
-                       P.graph_b != P.cur_b || P.graph_x != P.cur_x || P.graph_replace != P.replace_every;
-    if(!stale) return 0;
-    if(P.graph_mode != P.mode || P.graph_precond != P.precond || P.graph_b != P.cur_b || P.graph_x != P.cur_x ||
-       P.graph_replace != P.replace_every)
+    const bool stale = P.graph_mode != P.mode || P.graph_precond != P.precond || P.graph_b != P.cur_b ||
+                       P.graph_x != P.cur_x || P.graph_replace != P.replace_every || P.graph_routes != P.routes;
+    if(P.gexec[g] && !stale) return 0;
+    if(stale)
     {
         for(int k = 0; k < 2; ++k)
         {
@@ -333,6 +332,7 @@ static int ensure_graph(Problem& P, int g)
         P.graph_b = P.cur_b;
         P.graph_x = P.cur_x;
         P.graph_replace = P.replace_every;
+        P.graph_routes = P.routes;
     }
     HPCGX_HIP(hipStreamBeginCapture(P.s, hipStreamCaptureModeThreadLocal));
     int rc = enqueue_iteration(P, g == 1);

@@ -89,9 +89,11 @@ struct Problem
     int graph_mode = -1;
     bool graph_precond = true;
     int graph_replace = -1;
+    unsigned graph_routes = 0;
     CoarsePlan coarse[2];     // [precision]
     int coarse_rows = -1;     // levels of at most this many rows run in one workgroup (-1: COARSE_ROWS)
-    unsigned routes = 0;      // changes of what the kernels run on (Level::pat_off, coarse_rows), which plans hold
+    unsigned routes = 0;      // changes of what the kernels run on (Level::pat_off, exposed, coarse_rows), for
+                              // the graphs and the batch's plans that hold it
     RefPath* ref = nullptr;   // natural-order work vectors of the reference path (refpath.hip)
 
     // forget captured graphs (launch shapes or operands changed)
@@ -107,6 +109,13 @@ struct Problem
         graph_mode = -1;
     }
 };
+
+// Level::exposed
+inline void expose_columns(Problem& P, int l)
+{
+    if(!P.L[l].exposed) ++P.routes;
+    P.L[l].exposed = true;
+}
 
 int problem_create(Problem*& P, int nx, int ny, int nz, int nlevels, bool with_f64, bool with_mixed, hipStream_t s);
 void problem_destroy(Problem* P);
