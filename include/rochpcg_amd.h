@@ -327,6 +327,11 @@ int hpcgx_set_row_patterns(hpcgx_problem* p, int level, int on);
  * of the diagonal, or whose arrays hpcgx_level_arrays has handed out, is run as
  * launches whatever `rows` says.  Results do not depend on it. */
 int hpcgx_set_coarse_rows(hpcgx_problem* p, int rows);
+/* How a level is run at present: *patterns = the row patterns of its colour
+ * that has most, 0 where its columns are read from the array; *workgroup = 1
+ * where the V-cycle of precision `prec` (0 f64, 1 mixed) takes the level in one
+ * workgroup (no reference counterpart) */
+int hpcgx_get_routes(const hpcgx_problem* p, int prec, int level, int* patterns, int* workgroup);
 int hpcgx_synchronize(hpcgx_problem* p);
 int hpcgx_malloc(void** ptr, size_t bytes);
 int hpcgx_free(void* ptr);

@@ -92,6 +92,7 @@ def _load():
         "hpcgx_set_sweep_columns": ([vp, i32, i32], i32),
         "hpcgx_set_row_patterns": ([vp, i32, i32], i32),
         "hpcgx_set_coarse_rows": ([vp, i32], i32),
+        "hpcgx_get_routes": ([vp, i32, i32, P(i32), P(i32)], i32),
         "hpcgx_get_shape": ([vp, i32, i32, i32, P(i32), P(i32)], i32),
         "hpcgx_synchronize": ([vp], i32),
         "hpcgx_batch_create": ([i32, vp, i32, i32, vp, P(vp)], i32),
@@ -452,6 +453,13 @@ class Problem:
         """Largest level the V-cycle runs, with all below it, in one workgroup
         (-1: the default, 0: none; results do not change)."""
         _check(lib.hpcgx_set_coarse_rows(self.h, rows))
+
+    def get_routes(self, level, mixed=False):
+        """How a level is run: (row patterns of its colour that has most, 0 for
+        the column array; whether the V-cycle takes it in one workgroup)."""
+        n, w = C.c_int(), C.c_int()
+        _check(lib.hpcgx_get_routes(self.h, int(mixed), level, C.byref(n), C.byref(w)))
+        return n.value, bool(w.value)
 
     def get_shape(self, level, op, mixed=False):
         b, r = C.c_int(), C.c_int()

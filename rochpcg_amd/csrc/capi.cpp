@@ -661,6 +661,23 @@ int hpcgx_get_shape(const hpcgx_problem* p, int prec, int level, int op, int* bl
     return 0;
 }
 
+int hpcgx_get_routes(const hpcgx_problem* p, int prec, int level, int* patterns, int* workgroup)
+{
+    CHECK_P(p);
+    CHECK_LEVEL(p, level);
+    CHECK_PTRS(patterns, workgroup);
+    if(prec < 0 || prec > 1)
+    {
+        set_error("invalid precision");
+        return -2;
+    }
+    const Level& L = p->P->L[level];
+    const bool stored = prec == PREC_F64 ? p->P->has_f64 : p->P->has_mixed;
+    *patterns = L.use_pat() ? L.npat : 0;
+    *workgroup = stored && level >= coarse_first(*p->P, (Prec)prec);
+    return 0;
+}
+
 int hpcgx_synchronize(hpcgx_problem* p)
 {
     CHECK_P(p);
