@@ -516,11 +516,11 @@ static int build_plan(Problem& P, Prec prec)
                            prec == PREC_F64 ? 8 : 4, L.ell_col, L.desc, (uint16_t*)mem + cols[j]);
         HPCGX_HIP(hipGetLastError());
     }
-    std::vector<char> up(lay.bytes - lay.steps);
+    std::vector<char>& up = C.upload;
+    up.resize(lay.bytes - lay.steps);
     std::memcpy(up.data(), steps.data(), sizeof(CoarseStep) * steps.size());
     std::memcpy(up.data() + (lay.levels - lay.steps), h.data(), sizeof(CoarseLevel) * nc);
     HPCGX_HIP(hipMemcpyAsync(mem + lay.steps, up.data(), up.size(), hipMemcpyHostToDevice, P.s));
-    HPCGX_HIP(hipStreamSynchronize(P.s));
     C.lv = (CoarseLevel*)(mem + lay.levels);
     return 0;
 }

@@ -74,7 +74,8 @@ inline CoarseLayout coarse_layout(size_t ncolumns, size_t nsteps, size_t nlevels
     return o;
 }
 
-// build the plans of a problem whose levels and vectors exist
+// build the plans of a problem whose levels and vectors exist; they are complete,
+// and CoarsePlan::upload done with, when P.s has been waited for
 int coarse_build(Problem& P);
 void coarse_free(Problem& P);
 // the first level that runs in one workgroup, with everything below it

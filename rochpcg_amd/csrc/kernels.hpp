@@ -328,7 +328,7 @@ constexpr int slot_dim(int n) { return n > 0 ? n : 1; }
 // Why patterns: with f64 values a slot streams 12 B, 4 of them the column;
 // with f16 values 6 B, 4 of them the column -- yet the rows of a colour repeat
 // a handful of offset lists.  The patterns are found from the ELL itself at
-// setup (build_patterns), for whatever matrix it holds; a level whose rows
+// setup (scan_rows), for whatever matrix it holds; a level whose rows
 // repeat too little keeps its column array.  The offsets are exact, so both
 // sources give the same x values in the same slots and every sum is the same
 // bit for bit.
@@ -336,7 +336,7 @@ constexpr int slot_dim(int n) { return n > 0 ? n : 1; }
 // The colour's patterns (112 B each) are staged in LDS by the block while the
 // value loads are in flight, so the x gathers wait for one byte load and an
 // LDS read instead of for the whole column stream.  Gather offsets are 32-bit
-// byte offsets from x (one add-shift a slot); build_patterns keeps levels of
+// byte offsets from x (one add-shift a slot); scan_rows keeps levels of
 // 2^29 rows or more on the column array.
 template <bool PAT, int R, int BS>
 struct Cols;

@@ -539,17 +539,21 @@ struct ColorRanges
     int off[MAX_COLORS + 1];
 };
 constexpr uint8_t PAT_NONE = 255;   // no pattern yet
+constexpr int32_t NO_ROW = 0x7f7f7f7f;   // no row: equal bytes, so that a memset writes it
 static_assert(PAT_MAX < PAT_NONE, "pattern ids are one byte");
+static_assert(PAT_MAX % 8 == 0, "rounds are looked at by eight");
 
-// Window statistics of one colour's rows [off, off+size): the largest lower
-// count d, upper count W - us and last-colour count W - tl (stats[0..2]).
-__global__ __launch_bounds__(256) void k_window_stats(int64_t off, int64_t size, const int32_t* __restrict__ desc,
+// Window statistics of every colour (grid.y): the largest lower count d, upper
+// count W - us and last-colour count W - tl of its rows (stats[WIN_COUNT * c + kind]).
+__global__ __launch_bounds__(256) void k_window_stats(ColorRanges cr, const int32_t* __restrict__ desc,
                                                       int* __restrict__ stats)
 {
+    const int c = blockIdx.y;
+    const int64_t end = cr.off[c + 1];
     int mx[WIN_COUNT] = {0, 0, 0};
-    for(int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < size; i += (int64_t)gridDim.x * 256)
+    for(int64_t r = cr.off[c] + (int64_t)blockIdx.x * 256 + threadIdx.x; r < end; r += (int64_t)gridDim.x * 256)
     {
-        const int v = desc[off + i];
+        const int v = desc[r];
         mx[WIN_LOWER] = max(mx[WIN_LOWER], v & 255);
         mx[WIN_TAIL] = max(mx[WIN_TAIL], W - ((v >> 8) & 255));
         mx[WIN_UPPER] = max(mx[WIN_UPPER], W - ((v >> 16) & 255));
@@ -565,136 +569,141 @@ __global__ __launch_bounds__(256) void k_window_stats(int64_t off, int64_t size,
     __syncthreads();
     if(threadIdx.x == 0)
         for(int k = 0; k < WIN_COUNT; ++k)
-            atomicMax(stats + k, max(max(lmx[k][0], lmx[k][1]), max(lmx[k][2], lmx[k][3])));
+            atomicMax(stats + WIN_COUNT * c + k, max(max(lmx[k][0], lmx[k][1]), max(lmx[k][2], lmx[k][3])));
 }
 
-// Per colour, the slots a sweep thread loads per row of each window kind
-// (Level::win), from the row descriptors.
-static int window_stats(Level& L, hipStream_t s)
-{
-    const int nc = L.ncolors;
-    int* stats = nullptr;
-    HPCGX_HIP(hipMalloc(&stats, sizeof(int) * WIN_COUNT * nc));
-    HPCGX_HIP(hipMemsetAsync(stats, 0, sizeof(int) * WIN_COUNT * nc, s));
-    for(int c = 0; c < nc; ++c)
-    {
-        if(L.sizes[c] == 0) continue;
-        const int64_t g = std::min<int64_t>(1024, ceil_div(L.sizes[c], 256));
-        hipLaunchKernelGGL(k_window_stats, dim3((unsigned)g), dim3(256), 0, s, (int64_t)L.offsets[c],
-                           (int64_t)L.sizes[c], L.desc, stats + WIN_COUNT * c);
-        HPCGX_HIP(hipGetLastError());
-    }
-    std::vector<int> hs((size_t)WIN_COUNT * nc);
-    HPCGX_HIP(hipMemcpyAsync(hs.data(), stats, sizeof(int) * WIN_COUNT * nc, hipMemcpyDeviceToHost, s));
-    HPCGX_HIP(hipStreamSynchronize(s));
-    HPCGX_HIP(hipFree(stats));
-    for(int c = 0; c < nc; ++c)
-        for(int k = 0; k < WIN_COUNT; ++k) L.win[k][c] = (unsigned char)hs[WIN_COUNT * c + k];
-    return 0;
-}
-
-// One round of the pattern search: for every colour (grid.y) the first row
-// without a pattern, rep[c], stands for pattern `k`; its rows without one that
-// have the same offsets and descriptor get it, and next[c] becomes the first
-// row still without one (INT_MAX: none).
-__global__ __launch_bounds__(256) void k_pattern_round(ColorRanges cr, int k, const int32_t* __restrict__ col,
-                                                       const int32_t* __restrict__ desc,
-                                                       const int32_t* __restrict__ rep, int32_t* __restrict__ next,
+// Rounds [k0, k1) of the pattern search.  In round k the first row of every colour
+// (grid.y) without a pattern stands for pattern k; the colour's rows without one that
+// have the same offsets and descriptor get it, and first[k + 1] becomes the first row
+// still without one (NO_ROW: none; round 0 starts with the colour's first row).  More
+// than one round a launch where one block has the whole colour.
+template <int BS>
+__global__ __launch_bounds__(BS) void k_pattern_rounds(ColorRanges cr, int k0, int k1, const int32_t* __restrict__ col,
+                                                       const int32_t* __restrict__ desc, int32_t* first,
                                                        uint8_t* __restrict__ pat, int32_t* __restrict__ tab)
 {
-    const int c = blockIdx.y;
-    const int32_t q = rep[c];
-    if(q == INT_MAX) return;
+    const int c = blockIdx.y, nc = gridDim.y;
     const int64_t off = cr.off[c], end = cr.off[c + 1];
-    if(blockIdx.x == 0 && threadIdx.x <= W)
+    for(int k = k0; k < k1; ++k)
     {
-        const int p = threadIdx.x;
-        int32_t* t = tab + ((int64_t)c * PAT_MAX + k) * (PAT_QUADS * 4);
-        if(p == W)
-            t[p] = desc[q];
-        else
+        int32_t* next = first + (k + 1) * nc + c;
+        const int32_t q = k > 0 ? __hip_atomic_load(first + k * nc + c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+                                : (off < end ? (int32_t)off : NO_ROW);
+        if(q == NO_ROW) return;
+        if(blockIdx.x == 0 && threadIdx.x <= W)
         {
-            const int32_t v = col[ell_at(p, q)];
-            t[p] = v < 0 ? 0 : v - q;
+            const int p = threadIdx.x;
+            int32_t* t = tab + ((int64_t)c * PAT_MAX + k) * (PAT_QUADS * 4);
+            if(p == W)
+                t[p] = desc[q];
+            else
+            {
+                const int32_t v = col[ell_at(p, q)];
+                t[p] = v < 0 ? 0 : v - q;
+            }
         }
-    }
-    int first = INT_MAX;
-    const int32_t qd = desc[q];
-    for(int64_t r = off + (int64_t)blockIdx.x * 256 + threadIdx.x; r < end; r += (int64_t)gridDim.x * 256)
-    {
-        if(k > 0 && pat[r] != PAT_NONE) continue;
-        // every column at once: left to stop at the first that differs, the loads
-        // follow one another (eight rounds at 320^3 took 5 ms)
-        int32_t a[W];
-#pragma unroll
-        for(int p = 0; p < W; ++p) a[p] = col[ell_at(p, r)];
-        bool same = desc[r] == qd;
-#pragma unroll
-        for(int p = 0; p < W; ++p)
+        int left = NO_ROW;
+        const int32_t qd = desc[q];
+        for(int64_t r = off + (int64_t)blockIdx.x * BS + threadIdx.x; r < end; r += (int64_t)gridDim.x * BS)
         {
-            const int32_t b = col[ell_at(p, q)];
-            same &= ((a[p] < 0) == (b < 0)) & ((a[p] < 0) | (a[p] - (int32_t)r == b - q));
+            if(k > 0 && pat[r] != PAT_NONE) continue;
+            // every column at once: left to stop at the first that differs, the loads
+            // follow one another (eight rounds at 320^3 took 5 ms)
+            int32_t a[W];
+#pragma unroll
+            for(int p = 0; p < W; ++p) a[p] = col[ell_at(p, r)];
+            bool same = desc[r] == qd;
+#pragma unroll
+            for(int p = 0; p < W; ++p)
+            {
+                const int32_t b = col[ell_at(p, q)];
+                same &= ((a[p] < 0) == (b < 0)) & ((a[p] < 0) | (a[p] - (int32_t)r == b - q));
+            }
+            pat[r] = same ? (uint8_t)k : PAT_NONE;
+            if(!same && (int)r < left) left = (int)r;
         }
-        pat[r] = same ? (uint8_t)k : PAT_NONE;
-        if(!same && (int)r < first) first = (int)r;
+        for(int o = 32; o > 0; o >>= 1) left = min(left, __shfl_xor(left, o, 64));
+        // nearly every wave of the first round has such a row (the end of a line): look
+        // before the atomic, which one of a colour's first waves has made vain for the others
+        if((threadIdx.x & 63) == 0 && left < __hip_atomic_load(next, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+            atomicMin(next, left);
+        __syncthreads();
     }
-    for(int o = 32; o > 0; o >>= 1) first = min(first, __shfl_xor(first, o, 64));
-    // nearly every wave of the first round has such a row (the end of a line): look
-    // before the atomic, which one of a colour's first waves has made vain for the others
-    if((threadIdx.x & 63) == 0 && first < __hip_atomic_load(next + c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-        atomicMin(next + c, first);
 }
 
-// Row patterns of a level (Level::pat, Cols<true>) from its columns and
-// descriptors: at most PAT_MAX rounds over the rows, the first of which reads
+// Window statistics (Level::win: per colour, the slots a sweep thread loads per row)
+// and row patterns (Level::pat, Cols<true>) of a level, from its columns and
+// descriptors, with one look from the host.
+//
+// The patterns take at most PAT_MAX rounds over the rows, the first of which reads
 // every column once (0.8 ms at 320^3) and the others only rows still without a
-// pattern.  A level with a colour of more than PAT_MAX patterns (odd grids,
-// where the colours' sub-grids differ in size) keeps the column array alone; so
-// does one of 2^29 rows or more, whose f64 gather offsets exceed 32 bits.
-static int build_patterns(Level& L, hipStream_t s)
+// pattern; eight settle a parity colouring.  A level with a colour of more than
+// PAT_MAX patterns (odd grids, where the colours' sub-grids differ in size) keeps the
+// column array alone; so does one of 2^29 rows or more, whose f64 gather offsets
+// exceed 32 bits.
+//
+// A launch costs 2.3 us to queue and 5.5 us in a row of them, a look from the host
+// 21: colours of at most ONE_BLOCK_ROWS rows run eight rounds in one launch.  A
+// problem of 16^3, 32^3, 48^3 and 64^3 is created in 1.08, 1.25, 1.50 and 1.96 ms;
+// with a launch a round at every size in 1.27, 1.37, 1.67 and 2.07, and with one
+// block for colours of up to 32768 rows in 1.07, 1.25, 1.58 and 2.28.
+constexpr int ONE_BLOCK = 1024, ONE_BLOCK_ROWS = 4096;
+
+static int scan_rows(Level& L, hipStream_t s)
 {
     const int nc = L.ncolors;
-    if(L.m >= ((int64_t)1 << 29)) return 0;
-    // one allocation, the level's pattern numbers first: patterns, representatives
-    const size_t tab_at = ((size_t)L.m + 255) / 256 * 256, tab_bytes = sizeof(int32_t) * PAT_QUADS * 4 * PAT_MAX * nc;
-    const size_t rep_at = tab_at + tab_bytes;
-    DevTemp mem;
-    HPCGX_HIP(hipMalloc(&mem.p, rep_at + sizeof(int32_t) * nc * (PAT_MAX + 1)));
-    int32_t* tab = (int32_t*)((char*)mem.p + tab_at);
-    HPCGX_HIP(hipMemsetAsync(tab, 0, tab_bytes, s));
-    // the representatives of every round; round k + 1's are round k's `next`
-    std::vector<int32_t> rep((size_t)nc * (PAT_MAX + 1), INT_MAX);
+    const bool find = L.m < ((int64_t)1 << 29);
     ColorRanges cr;
     int mx = 0;
     for(int c = 0; c <= nc; ++c) cr.off[c] = L.offsets[c];
-    for(int c = 0; c < nc; ++c)
-    {
-        rep[c] = L.sizes[c] > 0 ? L.offsets[c] : INT_MAX;
-        mx = std::max(mx, L.sizes[c]);
-    }
-    int32_t* d = (int32_t*)((char*)mem.p + rep_at);
-    HPCGX_HIP(hipMemcpyAsync(d, rep.data(), sizeof(int32_t) * rep.size(), hipMemcpyHostToDevice, s));
+    for(int c = 0; c < nc; ++c) mx = std::max(mx, L.sizes[c]);
+    // statistics, then the first rows of every round
+    const size_t nstats = (size_t)WIN_COUNT * nc, nfirst = find ? (size_t)nc * (PAT_MAX + 1) : 0;
+    DevTemp scratch, mem;
+    HPCGX_HIP(hipMalloc(&scratch.p, sizeof(int32_t) * (nstats + nfirst)));
+    int32_t* stats = (int32_t*)scratch.p;
+    int32_t* first = stats + nstats;
+    HPCGX_HIP(hipMemsetAsync(stats, 0, sizeof(int32_t) * nstats, s));
     const dim3 grid((unsigned)std::min<int64_t>(1024, ceil_div(mx, 256)), (unsigned)nc);
-    for(int k = 0; k < PAT_MAX; ++k)
+    hipLaunchKernelGGL(k_window_stats, grid, dim3(256), 0, s, cr, L.desc, stats);
+    HPCGX_HIP(hipGetLastError());
+    // one allocation, the level's pattern numbers first
+    const size_t tab_at = ((size_t)L.m + 255) / 256 * 256, tab_bytes = sizeof(int32_t) * PAT_QUADS * 4 * PAT_MAX * nc;
+    if(find)
     {
-        hipLaunchKernelGGL(k_pattern_round, grid, dim3(256), 0, s, cr, k, L.ell_col, L.desc,
-                           (const int32_t*)d + (size_t)k * nc, d + (size_t)(k + 1) * nc, (uint8_t*)mem.p, tab);
-        HPCGX_HIP(hipGetLastError());
-        // eight rounds settle a parity colouring
-        if(k % 8 != 7) continue;
-        HPCGX_HIP(hipMemcpyAsync(rep.data(), d, sizeof(int32_t) * rep.size(), hipMemcpyDeviceToHost, s));
-        HPCGX_HIP(hipStreamSynchronize(s));
-        bool left = false;
-        for(int c = 0; c < nc; ++c) left = left || rep[(size_t)(k + 1) * nc + c] != INT_MAX;
-        if(left) continue;
-        L.npat = 0;
-        for(int j = 0; j <= k; ++j)
-            for(int c = 0; c < nc; ++c)
-                if(rep[(size_t)j * nc + c] != INT_MAX) L.npat = j + 1;
-        L.pat = (uint8_t*)mem.release();
-        L.pat_tab = tab;
-        return 0;
+        HPCGX_HIP(hipMalloc(&mem.p, tab_at + tab_bytes));
+        HPCGX_HIP(hipMemsetAsync((char*)mem.p + tab_at, 0, tab_bytes, s));
+        HPCGX_HIP(hipMemsetAsync(first, NO_ROW & 255, sizeof(int32_t) * nfirst, s));
     }
+    uint8_t* pat = (uint8_t*)mem.p;
+    int32_t* tab = (int32_t*)((char*)mem.p + tab_at);
+    std::vector<int32_t> h(nstats + nfirst);
+    bool done = !find;
+    for(int k0 = 0; k0 == 0 || (!done && k0 < PAT_MAX); k0 += 8)
+    {
+        if(find && mx <= ONE_BLOCK_ROWS)
+            hipLaunchKernelGGL(k_pattern_rounds<ONE_BLOCK>, dim3(1, nc), dim3(ONE_BLOCK), 0, s, cr, k0, k0 + 8, L.ell_col,
+                               L.desc, first, pat, tab);
+        else if(find)
+            for(int k = k0; k < k0 + 8; ++k)
+                hipLaunchKernelGGL(k_pattern_rounds<256>, grid, dim3(256), 0, s, cr, k, k + 1, L.ell_col, L.desc, first,
+                                   pat, tab);
+        HPCGX_HIP(hipGetLastError());
+        HPCGX_HIP(hipMemcpyAsync(h.data(), stats, sizeof(int32_t) * h.size(), hipMemcpyDeviceToHost, s));
+        HPCGX_HIP(hipStreamSynchronize(s));
+        if(done) break;
+        const int32_t* left = h.data() + nstats + (size_t)(k0 + 8) * nc;
+        done = std::all_of(left, left + nc, [](int32_t r) { return r == NO_ROW; });
+    }
+    for(int c = 0; c < nc; ++c)
+        for(int k = 0; k < WIN_COUNT; ++k) L.win[k][c] = (unsigned char)h[WIN_COUNT * c + k];
+    if(!find || !done) return 0;
+    L.npat = 1;
+    for(int k = 1; k < PAT_MAX; ++k)
+        for(int c = 0; c < nc; ++c)
+            if(h[nstats + (size_t)k * nc + c] != NO_ROW) L.npat = k + 1;
+    L.pat = (uint8_t*)mem.release();
+    L.pat_tab = tab;
     return 0;
 }
 
@@ -755,11 +764,10 @@ int build_level(Level& L, int nx, int ny, int nz, bool with_f64, bool with_f16, 
                            L.diag_h);
         HPCGX_HIP(hipGetLastError());
     }
-    HPCGX_HIP(hipStreamSynchronize(s));
+    HPCGX_TRY(scan_rows(L, s));   // waits for the stream
     HPCGX_HIP(hipFree(L.iperm_tmp));
     L.iperm_tmp = nullptr;
-    HPCGX_TRY(window_stats(L, s));
-    return build_patterns(L, s);
+    return 0;
 }
 
 int build_transfer(Level& F, Level& C, hipStream_t s)

@@ -19,6 +19,7 @@
 
 #include <cmath>
 #include <cstring>
+#include <mutex>
 
 namespace hpcgx
 {
@@ -29,6 +30,56 @@ static int alloc(void** p, size_t bytes)
     HPCGX_HIP(hipMalloc(p, bytes));
     return 0;
 }
+
+// Pinned host memory for the results that calls return (Problem::h_out), in slots of
+// a page that problems share: pinning a page costs 100-200 us where many are held
+// (64 pages 13 ms), an already pinned one nothing.  A page is freed with its last
+// slot.
+class PinnedSlots
+{
+public:
+    double* take()
+    {
+        std::lock_guard<std::mutex> hold(m);
+        for(Page& p : pages)
+            if(~p.used)
+            {
+                const int k = __builtin_ctzll(~p.used);
+                p.used |= 1ull << k;
+                return (double*)(p.mem + k * SLOT);
+            }
+        Page p;
+        if(hipHostMalloc((void**)&p.mem, SLOTS * SLOT, hipHostMallocPortable) != hipSuccess) return nullptr;
+        p.used = 1;
+        pages.push_back(p);
+        return (double*)p.mem;
+    }
+    void give(double* slot)
+    {
+        std::lock_guard<std::mutex> hold(m);
+        for(size_t i = 0; i < pages.size(); ++i)
+        {
+            const ptrdiff_t at = (char*)slot - pages[i].mem;
+            if(at < 0 || at >= (ptrdiff_t)(SLOTS * SLOT)) continue;
+            pages[i].used &= ~(1ull << (at / SLOT));
+            if(pages[i].used) return;
+            (void)hipHostFree(pages[i].mem);
+            pages.erase(pages.begin() + i);
+            return;
+        }
+    }
+
+private:
+    static constexpr size_t SLOTS = 64, SLOT = 64;   // 8 results each
+    struct Page
+    {
+        char* mem = nullptr;
+        uint64_t used = 0;
+    };
+    std::mutex m;
+    std::vector<Page> pages;
+};
+static PinnedSlots& pinned_slots = *new PinnedSlots;   // outlives every problem
 
 int problem_create(Problem*& out, int nx, int ny, int nz, int nlevels, bool with_f64, bool with_mixed, hipStream_t s)
 {
@@ -112,7 +163,8 @@ int problem_create(Problem*& out, int nx, int ny, int nz, int nlevels, bool with
        alloc((void**)&P->partial, sizeof(double) * P->partial_cap) ||
        alloc((void**)&P->dout, 8 * sizeof(double)) || alloc((void**)&P->ticket, sizeof(int)))
         return fail(-1);
-    if(hipHostMalloc((void**)&P->h_out, 8 * sizeof(double), hipHostMallocDefault) != hipSuccess)
+    P->h_out = pinned_slots.take();
+    if(!P->h_out)
     {
         set_error("hipHostMalloc failed");
         return fail(-1);
@@ -127,6 +179,7 @@ int problem_create(Problem*& out, int nx, int ny, int nz, int nlevels, bool with
         set_error("stream synchronisation failed after setup");
         return fail(-1);
     }
+    for(CoarsePlan& C : P->coarse) std::vector<char>().swap(C.upload);
     out = P;
     return 0;
 }
@@ -172,7 +225,7 @@ void problem_destroy(Problem* P)
     f(P->partial);
     f(P->dout);
     f(P->ticket);
-    if(P->h_out) (void)hipHostFree(P->h_out);
+    if(P->h_out) pinned_slots.give(P->h_out);
     if(P->own_stream && P->s) (void)hipStreamDestroy(P->s);
     delete P;
 }

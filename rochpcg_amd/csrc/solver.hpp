@@ -41,6 +41,7 @@ struct CoarsePlan
     size_t bytes = 0;              // of mem
     CoarseLevel* lv = nullptr;     // of level `first`
     size_t lds[MAX_LEVELS] = {};   // LDS of a run from each level
+    std::vector<char> upload;      // steps and descriptions on their way to mem (problem_create waits)
 };
 // Levels of at most this many rows run so, [precision].  One workgroup streams a
 // level's values at one CU's rate, launches at the GPU's: an iteration of 64^3,
