@@ -215,7 +215,8 @@ double hpcgx_flops_per_iteration(const hpcgx_problem* p);
 int hpcgx_iteration_bytes(const hpcgx_problem* p, int mode, double* vcycle_bytes, double* iteration_bytes);
 /* the same with each kernel's own loads: where a level has row patterns
  * (hpcgx_set_row_patterns) a slot counts its value alone and a row one byte
- * for its columns and descriptor */
+ * for its columns and descriptor (levels that run in one workgroup count alike,
+ * though they read 2 bytes a slot) */
 int hpcgx_stream_bytes(const hpcgx_problem* p, int mode, double* vcycle_bytes, double* iteration_bytes);
 
 /* ---- the reference's natural-order path on the device -------------------- */
@@ -273,6 +274,9 @@ int hpcgx_batch_cg(hpcgx_batch* b, int mode, int max_iter, double tolerance, int
  * (hpcgx_set_coarse_rows) counts as kind 1 -- kind_bytes[k] = their algorithmic HBM bytes per iteration,
  * *iter_ms = milliseconds per iteration (no reference counterpart) */
 int hpcgx_batch_profile(hpcgx_batch* b, int mode, int iters, double* kind_ms, double* kind_bytes, double* iter_ms);
+/* HBM bytes that the launches of one batched iteration load and store
+ * (hpcgx_stream_bytes for a batch; no reference counterpart) */
+int hpcgx_batch_stream_bytes(hpcgx_batch* b, int mode, double* bytes);
 /* residual history of problem k's last batched CG: normr after iterations
  * 0..niters into history (at most hist_len entries); *count = entries written */
 int hpcgx_batch_history(hpcgx_batch* b, int k, double* history, int hist_len, int* count);

@@ -103,6 +103,7 @@ def _load():
         "hpcgx_batch_cg": ([vp, i32, i32, f64, i32, vp, vp, vp], i32),
         "hpcgx_batch_history": ([vp, i32, vp, i32, P(i32)], i32),
         "hpcgx_batch_profile": ([vp, i32, i32, vp, vp, P(f64)], i32),
+        "hpcgx_batch_stream_bytes": ([vp, i32, P(f64)], i32),
         "hpcgx_malloc": ([P(vp), C.c_size_t], i32),
         "hpcgx_free": ([vp], i32),
         "hpcgx_memcpy_h2d": ([vp, vp, C.c_size_t], i32),
@@ -612,6 +613,12 @@ class Batch:
         out = {k: (ms[i] / iters, by[i]) for i, k in enumerate(self.BATCH_KINDS)}
         out["iteration"] = (it.value, float(by.sum()))
         return out
+
+    def stream_bytes(self, mode=CG_F64):
+        """Bytes that the launches of one iteration load and store."""
+        by = C.c_double()
+        _check(lib.hpcgx_batch_stream_bytes(self.h, mode, C.byref(by)))
+        return by.value
 
     def history(self, k, max_len=4097):
         """normr after iterations 0..niters of problem k's last batched CG."""

@@ -2,7 +2,7 @@
 // problems.  Each problem keeps its own hierarchy, vectors, reduction scratch
 // and CG scalars (a Problem); the V-cycle and the CG iteration are issued as
 // one launch per (operator, level, colour) covering every problem, so a whole
-// batched iteration is ~115 launches whatever the number of problems, and is
+// batched iteration is ~105 launches whatever the number of problems, and is
 // captured once as a hipGraph.  Blocks map to (problem, row block) through a
 // segment table in device memory (the segment records, then the segment of
 // every block); a problem's segments return at once after its own
@@ -358,6 +358,7 @@ struct Planner
                                       &P->sc->done));
             L.lds = std::max(L.lds, P->coarse[prec].lds[l]);
             L.bytes += vcycle_bytes(*P, l, prec != PREC_F64, false);
+            L.stream_bytes += vcycle_bytes(*P, l, prec != PREC_F64, true);
         }
         L.kind = BK_COARSE;
         L.prec = prec;
@@ -698,36 +699,37 @@ static int run_list(const std::vector<BLaunch>& v, hipStream_t s)
     return 0;
 }
 
-// algorithmic HBM bytes of one planned launch (the per-row model of
-// iteration_bytes in solver.hip by the ELL's bytes, over the launch's rows)
-static double launch_bytes(const BLaunch& L)
+// algorithmic HBM bytes of one planned launch (the per-row model of iteration_bytes
+// in solver.hip over the launch's rows): by the ELL's bytes, or (stream) what its
+// kernel loads
+static double launch_bytes(const BLaunch& L, bool stream)
 {
-    const bool f64 = L.prec == PREC_F64;
+    const bool f64 = L.prec == PREC_F64, pat = stream && L.pat;
     const double vb = f64 ? 8.0 : 2.0, xb = f64 ? 8.0 : 4.0, rb = L.r_f64 ? 8.0 : xb;
-    const double slot = 4.0 + vb, n = (double)L.nrows;
+    const double slot = vb + (pat ? 0.0 : 4.0), head = pat ? 1.0 : 4.0, full = stream ? head : 0.0, n = (double)L.nrows;
     const double zb = L.bf32 ? 4.0 : 8.0;
     switch(L.kind)
     {
-    case BK_SPMV: return n * (W * slot + 16.0);
-    case BK_FWD_ZERO: return n * (window_slots(L.win) * slot + 4.0 + vb + rb + xb);
-    case BK_BWD_ZERO: return n * (window_slots(L.win) * slot + 4.0 + vb + 2.0 * xb + (L.any_t ? xb : 0.0));
+    case BK_SPMV: return n * (W * slot + full + 16.0);
+    case BK_FWD_ZERO: return n * (window_slots(L.win) * slot + head + vb + rb + xb);
+    case BK_BWD_ZERO: return n * (window_slots(L.win) * slot + head + vb + 2.0 * xb + (L.any_t ? xb : 0.0));
     case BK_FWD_FULL:
         if(L.all_u)
         {
             int na = 0, nb = 0;
             window_pair_slots(L.win, L.win_tail, &na, &nb);
-            return n * ((na + nb) * slot + 4.0 + vb + rb + 3.0 * xb);
+            return n * ((na + nb) * slot + head + vb + rb + 3.0 * xb);
         }
-        return n * (W * slot + rb + xb + (L.any_t ? xb : 0.0));
-    case BK_BWD_FULL: return n * (window_slots(L.win) * slot + 4.0 + vb + 2.0 * xb);
-    case BK_RESTRICT: return n * (W * slot + rb + 8.0 + xb);
+        return n * (W * slot + full + rb + xb + (L.any_t ? xb : 0.0));
+    case BK_BWD_FULL: return n * (window_slots(L.win) * slot + head + vb + 2.0 * xb);
+    case BK_RESTRICT: return n * (W * slot + full + rb + 8.0 + xb);
     case BK_PROLONG: return n * (8.0 + 3.0 * xb);
     case BK_DOT: return n * (8.0 + zb);
     case BK_CG_P: return n * (zb + 16.0);
     case BK_CG_XR: return n * 48.0;
     case BK_COPY: return n * 16.0;
     case BK_WAXPBY: return n * 24.0;
-    case BK_COARSE: return L.bytes;
+    case BK_COARSE: return stream ? L.stream_bytes : L.bytes;
     }
     return 0.0;
 }
@@ -748,6 +750,24 @@ static int read_scalars(Batch& B, int slot)
     hipLaunchKernelGGL(kb_read_scalars, dim3((unsigned)ceil_div(n, 64)), dim3(64), 0, B.s, B.sc, n, B.h_sc + slot * n);
     HPCGX_HIP(hipGetLastError());
     HPCGX_HIP(hipEventRecord(B.read[slot], B.s));
+    return 0;
+}
+
+int batch_stream_bytes(Batch& B, int mode, double* bytes)
+{
+    if(mode != CG_F64 && mode != CG_MIXED)
+    {
+        set_error("invalid CG mode");
+        return -2;
+    }
+    HPCGX_TRY(ensure_plan(B));
+    if(B.iter[mode].empty())
+    {
+        set_error("the batch was built without the store this mode needs");
+        return -2;
+    }
+    *bytes = 0.0;
+    for(const BLaunch& L : B.iter[mode]) *bytes += launch_bytes(L, true);
     return 0;
 }
 
@@ -807,7 +827,7 @@ int batch_profile(Batch& B, int mode, int iters, double* kind_ms, double* kind_b
     double total = 0.0;
     if(!rc)
     {
-        for(size_t j = 0; j < nl; ++j) kind_bytes[kind_of(j)] += launch_bytes(it[j]);
+        for(size_t j = 0; j < nl; ++j) kind_bytes[kind_of(j)] += launch_bytes(it[j], false);
         for(int i = 0; i < iters; ++i)
         {
             hipEvent_t* E = ev.data() + (size_t)i * (nl + 1);

@@ -142,8 +142,8 @@ struct BLaunch
     int64_t nrows;    // rows (elements) over all segments
     int any_t;        // some segment keeps or reads SymGS partial sums (BSeg::t)
     CoarseRun* runs;  // BK_COARSE: device table of nseg runs, the LDS they take,
-    size_t lds;       // and their algorithmic bytes
-    double bytes;
+    size_t lds;       // and their algorithmic bytes, by the ELL's and as they are loaded
+    double bytes, stream_bytes;
 };
 
 static_assert(BK_COUNT == 12, "hpcgx_batch_profile reports 12 kinds");
@@ -185,5 +185,8 @@ int batch_cg(Batch& B, int mode, int max_iter, double tol, bool use_graph, int* 
 // iteration (each slot a kernel loads once, gathers from cache, own-row
 // vectors once), *iter_ms = milliseconds per iteration (first event to last)
 int batch_profile(Batch& B, int mode, int iters, double* kind_ms, double* kind_bytes, double* iter_ms);
+// HBM bytes that the launches of one iteration load and store (the byte model of
+// batch_profile, with row patterns where a launch reads them)
+int batch_stream_bytes(Batch& B, int mode, double* bytes);
 
 }  // namespace hpcgx

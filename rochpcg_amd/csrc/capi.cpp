@@ -811,6 +811,17 @@ int hpcgx_batch_profile(hpcgx_batch* b, int mode, int iters, double* kind_ms, do
     return batch_profile(*b->B, mode, iters, kind_ms, kind_bytes, iter_ms);
 }
 
+int hpcgx_batch_stream_bytes(hpcgx_batch* b, int mode, double* bytes)
+{
+    if(!b || !b->B)
+    {
+        set_error("null batch");
+        return -2;
+    }
+    CHECK_PTRS(bytes);
+    return batch_stream_bytes(*b->B, mode, bytes);
+}
+
 int hpcgx_batch_history(hpcgx_batch* b, int k, double* history, int hist_len, int* count)
 {
     if(!b || !b->B)
