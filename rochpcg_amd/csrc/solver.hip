@@ -49,7 +49,7 @@ public:
                 return (double*)(p.mem + k * SLOT);
             }
         Page p;
-        if(hipHostMalloc((void**)&p.mem, SLOTS * SLOT, hipHostMallocPortable) != hipSuccess) return nullptr;
+        if(hipHostMalloc((void**)&p.mem, SLOTS * SLOT, hipHostMallocDefault) != hipSuccess) return nullptr;
         p.used = 1;
         pages.push_back(p);
         return (double*)p.mem;
