@@ -569,26 +569,34 @@ __global__ __launch_bounds__(256) void k_window_stats(ColorRanges cr, const int3
     __syncthreads();
     if(threadIdx.x == 0)
         for(int k = 0; k < WIN_COUNT; ++k)
-            atomicMax(stats + WIN_COUNT * c + k, max(max(lmx[k][0], lmx[k][1]), max(lmx[k][2], lmx[k][3])));
+        {
+            // the first blocks have nearly always seen the largest already: an atomic of
+            // every block of 320^3 took 237 us
+            int* most = stats + WIN_COUNT * c + k;
+            const int v = max(max(lmx[k][0], lmx[k][1]), max(lmx[k][2], lmx[k][3]));
+            if(v > __hip_atomic_load(most, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(most, v);
+        }
 }
 
 // Rounds [k0, k1) of the pattern search.  In round k the first row of every colour
 // (grid.y) without a pattern stands for pattern k; the colour's rows without one that
 // have the same offsets and descriptor get it, and first[k + 1] becomes the first row
-// still without one (NO_ROW: none; round 0 starts with the colour's first row).  More
-// than one round a launch where one block has the whole colour.
+// still without one (NO_ROW: none).  Round 0 takes the colour's row `inner`, which on
+// the parity colourings lies inside the grid, so that the later rounds have the rows
+// at its faces left.  More than one round a launch where one block has the whole colour.
 template <int BS>
-__global__ __launch_bounds__(BS) void k_pattern_rounds(ColorRanges cr, int k0, int k1, const int32_t* __restrict__ col,
+__global__ __launch_bounds__(BS) void k_pattern_rounds(ColorRanges cr, int inner, int k0, int k1, const int32_t* __restrict__ col,
                                                        const int32_t* __restrict__ desc, int32_t* first,
                                                        uint8_t* __restrict__ pat, int32_t* __restrict__ tab)
 {
     const int c = blockIdx.y, nc = gridDim.y;
     const int64_t off = cr.off[c], end = cr.off[c + 1];
+    __shared__ int32_t wave_left[BS / 64];
     for(int k = k0; k < k1; ++k)
     {
         int32_t* next = first + (k + 1) * nc + c;
         const int32_t q = k > 0 ? __hip_atomic_load(first + k * nc + c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
-                                : (off < end ? (int32_t)off : NO_ROW);
+                                : (off < end ? (int32_t)min(off + inner, end - 1) : NO_ROW);
         if(q == NO_ROW) return;
         if(blockIdx.x == 0 && threadIdx.x <= W)
         {
@@ -623,10 +631,15 @@ __global__ __launch_bounds__(BS) void k_pattern_rounds(ColorRanges cr, int k0, i
             if(!same && (int)r < left) left = (int)r;
         }
         for(int o = 32; o > 0; o >>= 1) left = min(left, __shfl_xor(left, o, 64));
-        // nearly every wave of the first round has such a row (the end of a line): look
-        // before the atomic, which one of a colour's first waves has made vain for the others
-        if((threadIdx.x & 63) == 0 && left < __hip_atomic_load(next, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-            atomicMin(next, left);
+        if((threadIdx.x & 63) == 0) wave_left[threadIdx.x >> 6] = left;
+        __syncthreads();
+        if(threadIdx.x == 0)
+        {
+            for(int w = 1; w < BS / 64; ++w) left = min(left, wave_left[w]);
+            // nearly every block of the first round has such a row (the end of a line):
+            // look before the atomic, which one of the first has made vain for the others
+            if(left < __hip_atomic_load(next, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMin(next, left);
+        }
         __syncthreads();
     }
 }
@@ -636,8 +649,10 @@ __global__ __launch_bounds__(BS) void k_pattern_rounds(ColorRanges cr, int k0, i
 // descriptors, with one look from the host.
 //
 // The patterns take at most PAT_MAX rounds over the rows, the first of which reads
-// every column once (0.8 ms at 320^3) and the others only rows still without a
-// pattern; eight settle a parity colouring.  A level with a colour of more than
+// every column once (0.7 ms at 320^3) and the others only rows still without a
+// pattern (0.1-0.3 ms each; with the colour's first row, a corner of the grid, in
+// round 0 the rows inside waited for round 4, 4.9 ms in all against 2.8); eight
+// settle a parity colouring.  A level with a colour of more than
 // PAT_MAX patterns (odd grids, where the colours' sub-grids differ in size) keeps the
 // column array alone; so does one of 2^29 rows or more, whose f64 gather offsets
 // exceed 32 bits.
@@ -648,6 +663,9 @@ __global__ __launch_bounds__(BS) void k_pattern_rounds(ColorRanges cr, int k0, i
 // with a launch a round at every size in 1.27, 1.37, 1.67 and 2.07, and with one
 // block for colours of up to 32768 rows in 1.07, 1.25, 1.58 and 2.28.
 constexpr int ONE_BLOCK = 1024, ONE_BLOCK_ROWS = 4096;
+// blocks of a scan of larger levels: 1024 take 3.0 ms at 320^3 and 0.72 at 200x136x184,
+// 2048 2.9 and 0.82, 8192 2.8 and 0.87
+constexpr int SCAN_BLOCKS = 2048;
 
 static int scan_rows(Level& L, hipStream_t s)
 {
@@ -657,6 +675,7 @@ static int scan_rows(Level& L, hipStream_t s)
     int mx = 0;
     for(int c = 0; c <= nc; ++c) cr.off[c] = L.offsets[c];
     for(int c = 0; c < nc; ++c) mx = std::max(mx, L.sizes[c]);
+    const int inner = (int)(((int64_t)(L.nz / 4) * (L.ny / 2) + L.ny / 4) * (L.nx / 2) + L.nx / 4);
     // statistics, then the first rows of every round
     const size_t nstats = (size_t)WIN_COUNT * nc, nfirst = find ? (size_t)nc * (PAT_MAX + 1) : 0;
     DevTemp scratch, mem;
@@ -664,7 +683,7 @@ static int scan_rows(Level& L, hipStream_t s)
     int32_t* stats = (int32_t*)scratch.p;
     int32_t* first = stats + nstats;
     HPCGX_HIP(hipMemsetAsync(stats, 0, sizeof(int32_t) * nstats, s));
-    const dim3 grid((unsigned)std::min<int64_t>(1024, ceil_div(mx, 256)), (unsigned)nc);
+    const dim3 grid((unsigned)std::max<int64_t>(1, std::min<int64_t>(SCAN_BLOCKS / nc, ceil_div(mx, 256))), (unsigned)nc);
     hipLaunchKernelGGL(k_window_stats, grid, dim3(256), 0, s, cr, L.desc, stats);
     HPCGX_HIP(hipGetLastError());
     // one allocation, the level's pattern numbers first
@@ -682,11 +701,11 @@ static int scan_rows(Level& L, hipStream_t s)
     for(int k0 = 0; k0 == 0 || (!done && k0 < PAT_MAX); k0 += 8)
     {
         if(find && mx <= ONE_BLOCK_ROWS)
-            hipLaunchKernelGGL(k_pattern_rounds<ONE_BLOCK>, dim3(1, nc), dim3(ONE_BLOCK), 0, s, cr, k0, k0 + 8, L.ell_col,
+            hipLaunchKernelGGL(k_pattern_rounds<ONE_BLOCK>, dim3(1, nc), dim3(ONE_BLOCK), 0, s, cr, inner, k0, k0 + 8, L.ell_col,
                                L.desc, first, pat, tab);
         else if(find)
             for(int k = k0; k < k0 + 8; ++k)
-                hipLaunchKernelGGL(k_pattern_rounds<256>, grid, dim3(256), 0, s, cr, k, k + 1, L.ell_col, L.desc, first,
+                hipLaunchKernelGGL(k_pattern_rounds<256>, grid, dim3(256), 0, s, cr, inner, k, k + 1, L.ell_col, L.desc, first,
                                    pat, tab);
         HPCGX_HIP(hipGetLastError());
         HPCGX_HIP(hipMemcpyAsync(h.data(), stats, sizeof(int32_t) * h.size(), hipMemcpyDeviceToHost, s));
