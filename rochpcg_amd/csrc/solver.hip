@@ -373,6 +373,8 @@ static int ensure_graph(Problem& P, int g)
     if(P.gexec[g] && !stale) return 0;
     if(stale)
     {
+        // a graph that is replaced between iterations may still be running
+        if(P.gexec[0] || P.gexec[1]) HPCGX_HIP(hipStreamSynchronize(P.s));
         for(int k = 0; k < 2; ++k)
         {
             if(P.gexec[k]) (void)hipGraphExecDestroy(P.gexec[k]);

@@ -137,3 +137,20 @@ def test_drop_in_layer(hip, tmp_path):
     out = subprocess.run([exe], capture_output=True, text=True, timeout=60)
     assert out.returncode == 0, out.stdout + out.stderr
     assert out.stdout.split() == ["26", "26"]
+
+
+def test_written_between_iterations(hip):
+    """Pointers taken while iterations are queued: the graph is replaced behind them."""
+    out = []
+    for use_graph in (True, False):
+        G = hip.Problem(32, 24, 16, nlevels=4, stores=hip.STORE_F64)
+        G.make_rhs(1, 31)
+        G.cg_begin(max_iter=8)
+        G.cg_iterate(4, use_graph=use_graph)
+        V = G.level_views(0)
+        col = V["ell_col"].host()
+        V["ell_col"].upload(col)   # the same columns, read in place from here
+        G.cg_iterate(4, use_graph=use_graph)
+        out.append(G.cg_end(hist_len=9)["history"])
+        G.close()
+    assert np.array_equal(*out) and len(out[0]) == 9
