@@ -17,8 +17,8 @@
 // has come out as NaN, the V-cycle is run again over the used slots alone (CM_USED).
 //
 // Measured, a CG iteration of FP64 / mixed with every level as launches and with
-// its coarse levels here: 16^3 254 / 238 -> 148 / 114 us, 32^3 282 / 254 ->
-// 220 / 171 us, 64^3 382 / 313 -> 358 / 268 us, 104^3 561 / 418 -> 545 / 391 us;
+// its coarse levels here: 16^3 253 / 238 -> 139 / 115 us, 32^3 279 / 257 ->
+// 212 / 176 us, 64^3 380 / 315 -> 355 / 267 us, 104^3 562 / 421 -> 547 / 393 us;
 // a step takes 0.5-0.9 us.
 //
 // Per row the arithmetic is that of the row_* functions of kernels.hpp, on the same
