@@ -23,13 +23,13 @@
 namespace hpcgx
 {
 
-// the fold of a reducing launch: block k folds the partials of segment k's
-// problem (one per block of the problem's segments) if k is its first segment
+// the fold of a reducing launch, a block a problem: it folds the partials of the
+// problem's segments (one per block of theirs), the first of which is folds[k]
 template <int BS>
-__global__ __launch_bounds__(BS) void kb_fold(const BSeg* __restrict__ segs)
+__global__ __launch_bounds__(BS) void kb_fold(const BSeg* __restrict__ segs, const int32_t* __restrict__ folds)
 {
-    const BSeg& S = segs[blockIdx.x];
-    if(gated(S.gate) || S.ra.partial == nullptr || S.nfold == 0) return;
+    const BSeg& S = segs[folds[blockIdx.x]];
+    if(gated(S.gate)) return;
     fold_partials<BS>(S.ra.partial, S.nfold, S.ra);
 }
 
@@ -187,7 +187,7 @@ static int launch(const BLaunch& L, hipStream_t s)
     HPCGX_HIP(hipGetLastError());
     if(L.kind == BK_DOT || L.kind == BK_CG_XR || (L.kind == BK_SPMV && L.dot))
     {
-        hipLaunchKernelGGL((kb_fold<FOLD_THREADS>), dim3((unsigned)L.nseg), dim3(FOLD_THREADS), 0, s, L.segs);
+        hipLaunchKernelGGL((kb_fold<FOLD_THREADS>), dim3((unsigned)L.nfolds), dim3(FOLD_THREADS), 0, s, L.segs, L.folds);
         HPCGX_HIP(hipGetLastError());
     }
     return 0;
@@ -267,11 +267,13 @@ struct Planner
         L.nseg = (int)nseg;
         L.nblocks = assign_blocks(segs, nseg, L.block, vector_kind, L.rows);
         L.pat = L.kind <= BK_RESTRICT;
+        std::vector<int32_t> folds;
         // the segments of a problem follow each other: their partials too, and
         // the first folds them all
         for(size_t j = 0, first = 0; j < nseg; ++j)
         {
             if(prob[j] != prob[first]) first = j;
+            if(j == first && segs[j].ra.partial) folds.push_back((int32_t)j);
             segs[j].part0 = segs[first].nfold;
             segs[first].nfold += segs[j].nblk;
             if(segs[j].ra.partial && segs[first].nfold > B.probs[prob[j]]->partial_cap)
@@ -283,10 +285,15 @@ struct Planner
             L.nrows += segs[j].size;
             if(segs[j].t) L.any_t = 1;
         }
-        std::vector<char> h(table_bytes(nseg, L.nblocks));
+        // the folds lie behind the map, whose last word seg_of reads whole
+        const size_t folds_at = (table_bytes(nseg, L.nblocks) + 3) / 4 * 4;
+        std::vector<char> h(folds_at + sizeof(int32_t) * folds.size());
         std::memcpy(h.data(), segs, sizeof(BSeg) * nseg);
         block_map(segs, nseg, reinterpret_cast<uint16_t*>(h.data() + sizeof(BSeg) * nseg));
-        HPCGX_HIP(hipMalloc((void**)&L.segs, h.size() + 2));   // seg_of reads whole words of the map
+        if(!folds.empty()) std::memcpy(h.data() + folds_at, folds.data(), sizeof(int32_t) * folds.size());
+        HPCGX_HIP(hipMalloc((void**)&L.segs, h.size()));
+        L.folds = (const int32_t*)((const char*)L.segs + folds_at);
+        L.nfolds = (int)folds.size();
         B.tables.push_back(L.segs);
         HPCGX_HIP(hipMemcpy(L.segs, h.data(), h.size(), hipMemcpyHostToDevice));
         out->push_back(L);

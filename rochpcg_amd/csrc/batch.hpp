@@ -138,6 +138,8 @@ struct BLaunch
     int nseg;
     int64_t nblocks;
     BSeg* segs;       // device table
+    const int32_t* folds;   // reductions: each problem's first segment, in that table
+    int nfolds;
     double alpha, beta;
     int64_t nrows;    // rows (elements) over all segments
     int any_t;        // some segment keeps or reads SymGS partial sums (BSeg::t)
